@@ -60,6 +60,21 @@ def smoother_colour_values(dim: int, k: int, level: int):
     return out
 
 
+def smoother_row_values(k: int, level: int):
+    """Algorithmic values moved by each launch of one 3D multiplicative sweep
+    with the row kernel (both x colours of one y and z parity): b read on the
+    interiors of the rows plus u read or written once on the rows' boxes."""
+    n = 1 << level
+    N1 = k * n + 1
+    out = []
+    for c in range(4):
+        py, pz = (n - (c & 1)) // 2, (n - (c >> 1)) // 2
+        if py and pz:
+            out.append((N1 - 2) * py * (2 * k - 1) * pz * (2 * k - 1)
+                       + N1 * (2 * k * py + 1) * (2 * k * pz + 1))
+    return out
+
+
 def measured_traffic(kernel: str, dim: int, k: int, level: int):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 --pmc
     summary (profiles/traffic.json: FETCH_SIZE and WRITE_SIZE runs, each
@@ -78,19 +93,11 @@ def measured_traffic(kernel: str, dim: int, k: int, level: int):
 
 
 def dominant_kernel_name(core, dim: int, k: int, level: int) -> str:
-    """Name of the FP32 smoother kernel a finest-level colour launch runs
-    with the current tuning (3D k <= 3: the patch-group kernel)."""
-    if dim == 3 and k <= 3:
-        n = 1 << level
-        patches = (n // 2) ** 3
-        npw = 1
-        if patches > core.get_tuning("group_min_patches"):
-            npw = core.get_tuning("patches_per_wave")
-        waves = core.get_tuning("group_waves") if npw <= 2 else 1
-        if waves == 0:
-            waves = 4  # automatic: 4 wavefronts per work-group in FP32
-        return f"patch3d_group_kernel<{k}, float, 0, {npw}, {waves}>"
-    return f"patch3d_kernel<{k}, float, false>"
+    """Name of the FP32 smoother kernel a finest-level launch runs with the
+    default tuning (3D k = 3: the row kernel's chunk and work-group size)."""
+    if dim == 3 and k == 3:
+        return f"patch_rows3d_kernel<3, float, false, 16, {256 if level >= 6 else 512}>"
+    return f"patch_rows3d_kernel<{k}, float" if dim == 3 else f"patch2d_kernel<{k}, float, false>"
 
 
 def _best_ms(fn, reps):
@@ -201,9 +208,9 @@ def mfma_flops_per_patch(k: int) -> int:
 
 
 def mfma_report(core, ctx, k, level, reps):
-    """Finest-level colour pass of the FP32 smoother with the matrix-core
-    kernel and with the LDS/FMA kernel (eager launches, best of reps x 8
-    colours); MFMA utilisation = issued matrix-core FLOPs / time / the
+    """Finest-level colour pass of the FP32 smoother with the row kernel (the
+    default; half a launch), the matrix-core kernel and the LDS/FMA kernel
+    (eager launches, best of reps x 8 colours); MFMA utilisation = issued matrix-core FLOPs / time / the
     157.3 TFLOP/s dense FP32 matrix peak."""
     import torch
     op = core.LaplaceOperator(ctx, 3, k, level, torch.float32)
@@ -214,17 +221,20 @@ def mfma_report(core, ctx, k, level, reps):
     n = 1 << level
     patches = (n - 1) ** 3
     res = {}
+    res["rows"] = _best_ms(lambda: sm.step(u, b), max(3, reps)) * 1e3 / 8
     for mf in (1, 0):
-        prev = core.set_tuning("mfma_smoother", mf)
+        prev = core.set_tuning("mfma_smoother", mf), core.set_tuning("row_sweeps", 0)
         try:
             ms = _best_ms(lambda: sm.step(u, b), max(3, reps))
         finally:
-            core.set_tuning("mfma_smoother", prev)
+            core.set_tuning("mfma_smoother", prev[0])
+            core.set_tuning("row_sweeps", prev[1])
         res["mfma" if mf else "fma"] = ms * 1e3 / 8
     fl = mfma_flops_per_patch(k) * patches
     ach = fl / (res["mfma"] * 8 * 1e-6) / 1e12
     waves = core.get_tuning("mfma_waves")  # wavefronts per patch
     return {"kernel": f"patch3d_mfma_kernel<{k}, {waves}>",
+            "us_per_colour_rows": round(res["rows"], 2),
             "us_per_colour_mfma": round(res["mfma"], 2),
             "us_per_colour_lds_fma": round(res["fma"], 2), "issued_TFLOPs": round(ach, 1),
             "peak_TFLOPs": 157.3, "frac": round(ach / 157.3, 3),
@@ -259,14 +269,15 @@ def hbm_report(core, ctx, k, level, reps):
         y = torch.empty_like(u)
         if s == 4:
             for mf in (1, 0):
-                prev = core.set_tuning("mfma_smoother", mf)
+                prev = core.set_tuning("mfma_smoother", mf), core.set_tuning("row_sweeps", 0)
                 try:
                     rate(f"smoother_colour_fp32_{'mfma' if mf else 'lds_fma'}",
                          lambda: sm.step(u, b), s * sum(vals), len(vals))
                 finally:
-                    core.set_tuning("mfma_smoother", prev)
-        else:
-            rate("smoother_colour_fp64", lambda: sm.step(u, b), s * sum(vals), len(vals))
+                    core.set_tuning("mfma_smoother", prev[0])
+                    core.set_tuning("row_sweeps", prev[1])
+        rows = smoother_row_values(k, level)
+        rate(f"smoother_rows_{tag}", lambda: sm.step(u, b), s * sum(rows), len(rows))
         rate(f"vmult_{tag}", lambda: op.vmult(y, u), 2 * s * op.n_dofs, 1)
         rate(f"residual_{tag}", lambda: op.residual(y, b, u), 3 * s * op.n_dofs, 1)
         tr = core.MGTransferCUDA(ctx, 3, k, 1, level, dt)
@@ -643,7 +654,11 @@ def kernel_bench(args):
         u = torch.rand(op.n_dofs, generator=g, device="cuda:0", dtype=dt)
         b = torch.rand(op.n_dofs, generator=g, device="cuda:0", dtype=dt)
         tag = "fp32" if s == 4 else "fp64"
-        timed(f"smoother_colour_{tag}", lambda: sm.step(u, b), s * sum(vals), len(vals))
+        if dim == 3:
+            rows = smoother_row_values(k, level)
+            timed(f"smoother_rows_{tag}", lambda: sm.step(u, b), s * sum(rows), len(rows))
+        else:
+            timed(f"smoother_colour_{tag}", lambda: sm.step(u, b), s * sum(vals), len(vals))
         if dim == 3 and k <= 3:
             # patch-group kernel at 1, 2 and 4 patches per wavefront
             prev_min = core.set_tuning("group_min_patches", 0)
@@ -815,11 +830,11 @@ def main():
     mg32, r32 = run(torch.float32, args.steps, args.warmup, True)
     value = N / (r32["ms"] / 1e3) / 1e6
 
-    # dominant kernel: finest-level patch-smoother colour launch (FP32)
+    # dominant kernel: finest-level patch-smoother launch (FP32)
     cnt, tot_ms = r32["profile"]["smooth_fine"]
-    vals = smoother_colour_values(dim, k, level)
-    # each sweep launches every colour once; bytes per launch averaged over
-    # the colours of a sweep
+    vals = smoother_row_values(k, level) if dim == 3 else smoother_colour_values(dim, k, level)
+    # bytes per launch averaged over the launches of a sweep (3D: four, two
+    # colours each)
     bytes_per_launch = 4.0 * sum(vals) / len(vals)
     avg_launch_ms = tot_ms / max(cnt, 1)
     achieved = bytes_per_launch / (avg_launch_ms * 1e-3) / 1e9
@@ -828,7 +843,8 @@ def main():
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic,
-                "kernel": f"{kernel_name} (finest-level colour launch)",
+                "kernel": f"{kernel_name} (finest-level launch"
+                          f"{', two colours' if dim == 3 else ''})",
                 "avg_launch_us": round(avg_launch_ms * 1e3, 2), "launches": cnt,
                 "algorithmic_bytes_per_launch": round(bytes_per_launch)}
 

@@ -231,6 +231,19 @@ namespace
     virtual ~LaunchTimer()                     = default;
   };
 
+  // 3D multiplicative sweeps take the row kernel (two colours per launch)
+  // unless it is switched off or a knob of the per-colour kernels was changed
+  bool
+  row_sweeps_on()
+  {
+    const Tuning t, &c = tuning();
+    return c.row_sweeps != 0 && c.small_colour_patches == t.small_colour_patches &&
+           c.group_min_patches == t.group_min_patches &&
+           c.patches_per_wave == t.patches_per_wave && c.group_waves == t.group_waves &&
+           c.row_staged == t.row_staged && c.mfma_smoother == t.mfma_smoother &&
+           c.mfma_waves == t.mfma_waves;
+  }
+
   // one smoothing sweep; `resid` is level-sized scratch for the additive
   // form.  from_zero: u is taken as zero on entry (vmult semantics); the
   // forward multiplicative sweep then starts with the colour-0 pass that
@@ -276,6 +289,20 @@ namespace
         return;
       }
     const long e = timer ? timer->tic_launch() : -1;
+    if (lvl->dim == 3 && row_sweeps_on())
+      {
+        // two colours per launch
+        const bool rev = variant == GTPS_MULT_REV;
+        for (int cc = 0; cc < 4; ++cc)
+          {
+            const int c = rev ? 3 - cc : cc;
+            launch_patch_rows(lvl, u, b, c & 1, c >> 1, rev ? 1 : 0,
+                              from_zero && !rev && cc == 0, relax);
+          }
+        if (timer)
+          timer->toc_launch(e, 4);
+        return;
+      }
     for (int cc = 0; cc < ncol; ++cc)
       {
         const int c = variant == GTPS_MULT_REV ? ncol - 1 - cc : cc;
@@ -1900,6 +1927,12 @@ extern "C"
           prev                   = tuning().mfma_smoother;
           tuning().mfma_smoother = (int)value;
         }
+      else if (k == "row_sweeps")
+        {
+          GTPS_REQUIRE(value == 0 || value == 1, "row_sweeps must be 0 or 1");
+          prev                = tuning().row_sweeps;
+          tuning().row_sweeps = (int)value;
+        }
       else if (k == "mfma_waves")
         {
           GTPS_REQUIRE(value == 4 || value == 8 || value == 16,
@@ -1939,6 +1972,8 @@ extern "C"
         v = tuning().mfma_smoother;
       else if (k == "mfma_waves")
         v = tuning().mfma_waves;
+      else if (k == "row_sweeps")
+        v = tuning().row_sweeps;
       else if (k == "vmult_zdiv")
         v = tuning().vmult_zdiv;
       else if (k == "vmult_tile")

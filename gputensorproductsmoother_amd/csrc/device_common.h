@@ -52,7 +52,18 @@ namespace gtps
     static constexpr int SE      = lamInv2 + NI * NI;
     static constexpr int SO      = SE + (MH + 1) * NE;
     static constexpr int lamInv3p = SO + (MH > 0 ? MH * NO : 0);
-    static constexpr int size    = lamInv3p + NI * NI * NI;
+    // Face form of the patch solve (even/odd numbering).  IE/IO hold S^T M
+    // of the interior (the map nodal -> eigen coordinates, S^{-1}) by folded
+    // node rows like SE/SO; mv = S^T M e_0 couples the left end node (the
+    // right end has the same entry for an even vector, the opposite one for
+    // an odd vector) and at = S^T K e_0 - lambda mv its stiffness once the
+    // end's basis function is made M-orthogonal to the interior.
+    // (lamInv3p, mv and at are contiguous: one block of per-lane operands.)
+    static constexpr int mv   = lamInv3p + NI * NI * NI;
+    static constexpr int at   = mv + NI;
+    static constexpr int IE   = at + NI;
+    static constexpr int IO   = IE + (MH + 1) * NE;
+    static constexpr int size = IO + (MH > 0 ? MH * NO : 0);
   };
 
   // Column range of row r of a 2-cell patch matrix (block sparsity: rows
@@ -137,6 +148,69 @@ namespace gtps
   {
     return (__umulhi(n, f.m) + n) >> f.s;
   }
+
+      // Fast-diagonalisation transforms in the even/odd eigenbasis (tables
+      // Tab::SE, Tab::SO): t = S^T v with t numbered even vectors first, and
+      // its inverse v = S t.  The reflection symmetry of the eigenvectors
+      // halves the products: K(K) + (K-1)^2 multiply-adds and 2(K-1)
+      // additions instead of (2K-1)^2.
+      template <int K, typename T>
+      __device__ __forceinline__ void
+      fd_fwd(const T *SE, const T *SO, const T (&v)[2 * K - 1], T (&t)[2 * K - 1])
+      {
+        constexpr int NI = 2 * K - 1, MH = K - 1, NE = K, NO = K - 1;
+        T e[MH + 1], o[MH > 0 ? MH : 1];
+  #pragma unroll
+        for (int i = 0; i < MH; ++i)
+          {
+            e[i] = v[i] + v[NI - 1 - i];
+            o[i] = v[i] - v[NI - 1 - i];
+          }
+        e[MH] = v[MH];
+  #pragma unroll
+        for (int q = 0; q < NE; ++q)
+          {
+            T s = 0;
+  #pragma unroll
+            for (int i = 0; i <= MH; ++i)
+              s += SE[i * NE + q] * e[i];
+            t[q] = s;
+          }
+  #pragma unroll
+        for (int q = 0; q < NO; ++q)
+          {
+            T s = 0;
+  #pragma unroll
+            for (int i = 0; i < MH; ++i)
+              s += SO[i * NO + q] * o[i];
+            t[NE + q] = s;
+          }
+      }
+
+      template <int K, typename T>
+      __device__ __forceinline__ void
+      fd_inv(const T *SE, const T *SO, const T (&t)[2 * K - 1], T (&v)[2 * K - 1])
+      {
+        constexpr int NI = 2 * K - 1, MH = K - 1, NE = K, NO = K - 1;
+  #pragma unroll
+        for (int i = 0; i < MH; ++i)
+          {
+            T pe = 0, po = 0;
+  #pragma unroll
+            for (int q = 0; q < NE; ++q)
+              pe += SE[i * NE + q] * t[q];
+  #pragma unroll
+            for (int q = 0; q < NO; ++q)
+              po += SO[i * NO + q] * t[NE + q];
+            v[i]          = pe + po;
+            v[NI - 1 - i] = pe - po;
+          }
+        T pm = 0;
+  #pragma unroll
+        for (int q = 0; q < NE; ++q)
+          pm += SE[MH * NE + q] * t[q];
+        v[MH] = pm;
+      }
 
   __device__ __forceinline__ int
   linear_block_id()

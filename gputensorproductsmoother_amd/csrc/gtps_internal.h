@@ -244,6 +244,13 @@ namespace gtps
     // 1 = 8x8 / 256, 2 = 16x8 / 256; 3: by precision.  k = 7: 0 = 8x2 /
     // 512, 1 = 4x4 / 1024, 2 and 3 = 4x4 / 512
     int       vmult_tile = 3;
+    // 3D multiplicative sweeps: 1 = row kernel, two colours per launch; 0 =
+    // the per-colour kernels.  Measured on MI355X (us per sweep, row /
+    // per-colour): Q1 128^3 FP32 43 / 272, Q2 128^3 209 / 413, Q3 64^3 98 /
+    // 168 and FP64 156 / 252, Q4 32^3 55 / 377, Q5 32^3 FP64 191 / 599, Q7
+    // 32^3 262 / 542 and FP64 568 / 2746; smallest gains on coarse levels
+    // (Q3 8^3 23 / 32, Q7 8^3 64 / 68).
+    int       row_sweeps = 1;
     // bumped by every successful gtps_set_tuning: HIP graphs captured under
     // an older generation are re-captured before their next replay
     unsigned long long generation = 0;
@@ -268,6 +275,12 @@ namespace gtps
   // sum_i x_i y_i written per block to ctx->ws.partials; returns #blocks.
   int launch_laplace(const gtps_level *lvl, void *y, const void *x,
                      const void *b, bool fused_dot);
+
+  // smoother_row.hip: colours (first, py, pz) and then (1 - first, py, pz) of
+  // the 3D multiplicative sweep in one launch; zero: u = 0 on entry (needs
+  // first = 0, py = pz = 0)
+  void launch_patch_rows(const gtps_level *lvl, void *u, const void *src,
+                         int py, int pz, int first, bool zero, double relax);
 
   // coeff.hip: variable-coefficient operator (3D). y = A(c) x (resid:
   // y = b - A(c) x; transpose: y = A(c)^T x); a null level coefficient

@@ -373,6 +373,26 @@ namespace gtps
           for (int a = 0; a < NI; ++a)
             tab[TB::lamInv3p + (c * NI + b2) * NI + a] =
               1.0 / (b.lam[perm[c]] + b.lam[perm[b2]] + b.lam[perm[a]]);
+      // face form: S^T M and S^T K applied to the patch nodes
+      const int NP    = 2 * K + 1;
+      auto      sproj = [&](const std::vector<double> &A, int node, int j) {
+        double s = 0.0;
+        for (int r = 0; r < NI; ++r)
+          s += b.S[r * NI + j] * A[(r + 1) * NP + node];
+        return s;
+      };
+      for (int i = 0; i <= TB::MH; ++i)
+        for (int e = 0; e < TB::NE; ++e)
+          tab[TB::IE + i * TB::NE + e] = sproj(b.patchM, i + 1, even[e]);
+      for (int i = 0; i < TB::MH; ++i)
+        for (int o = 0; o < TB::NO; ++o)
+          tab[TB::IO + i * TB::NO + o] = sproj(b.patchM, i + 1, odd[o]);
+      for (int q = 0; q < NI; ++q)
+        {
+          const double m  = sproj(b.patchM, 0, perm[q]);
+          tab[TB::mv + q] = m;
+          tab[TB::at + q] = sproj(b.patchK, 0, perm[q]) - b.lam[perm[q]] * m;
+        }
       return tab;
     }
 

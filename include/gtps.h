@@ -114,6 +114,14 @@ const char *gtps_version(void);
  *                           degree 4..7 runs its 1D contractions on the
  *                           matrix cores (v_mfma_f32_16x16x4f32, patches
  *                           padded to 16^3); 0: the LDS/FMA kernel.
+ *   "row_sweeps"            1 (default): 3D multiplicative sweeps smooth the
+ *                           two colours of equal y and z parity in one
+ *                           launch, one work-group per x-row of patches;
+ *                           0, or any other value than the default of
+ *                           small_colour_patches, group_min_patches,
+ *                           patches_per_wave, group_waves, row_staged,
+ *                           mfma_smoother or mfma_waves: one launch per
+ *                           colour with the kernels these knobs choose;
  *   "mfma_waves"            matrix-core smoother wavefronts per patch: 4,
  *                           8 (default) or 16.
  * Results do not depend on the knobs beyond round-off.  No reference

@@ -231,6 +231,50 @@ def test_smoother_both_kernel_paths(core, ctx, dim, k, level, variant, prec, pat
     assert rel_err(ud.cpu().numpy(), ref) < tol
 
 
+# one patch; fewer patches than a chunk; several chunks with a short last one
+# (chunks hold 64, 32, 16, 8, 6/5, 4, 4/3 patches of one x parity, k = 1..7)
+ROW_CASES = [(1, 2), (1, 8), (2, 1), (2, 7), (3, 1), (3, 2), (3, 5), (3, 6), (4, 2), (4, 5),
+             (5, 2), (5, 4), (6, 3), (6, 4), (7, 1), (7, 3), (7, 4)]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("variant", ["fwd", "rev", "zero"])
+@pytest.mark.parametrize("k,level", ROW_CASES)
+def test_smoother_row_kernel(core, ctx, k, level, variant, prec):
+    """The row kernel (two colours per launch, rows walked in chunks) on a
+    general state with boundary values and damping, and from zero, against
+    the oracle's sweep; the per-colour kernels agree as well."""
+    if level >= 7 and (variant == "rev" or prec == "fp64"):
+        pytest.skip("17M DoFs: one precision and two orders")
+    _announce("smoother-rows", k, level, variant, prec)
+    g = rng(level * 11 + k)
+    N = n_dofs(3, k, level)
+    b, u = g.uniform(-1, 1, (2, N))
+    if prec == "fp32":
+        u = u.astype(np.float32).astype(np.float64)
+        b = b.astype(np.float32).astype(np.float64)
+    relax = 0.75
+    ov = O.MULT_REV if variant == "rev" else O.MULT_FWD
+    ref = O.smoother_step(3, k, level, b, np.zeros(N) if variant == "zero" else u, variant=ov,
+                          relax=relax)
+    op = core.LaplaceOperator(ctx, 3, k, level, _dt(prec))
+    sm = core.PatchSmoother(op, core.PatchSmoother.MULTIPLICATIVE_REVERSE if variant == "rev"
+                            else core.PatchSmoother.MULTIPLICATIVE, relax)
+    out = []
+    for rows in (1, 0):
+        prev = core.set_tuning("row_sweeps", rows)
+        try:
+            ud = _to_dev(u, prec)
+            (sm.vmult if variant == "zero" else sm.step)(ud, _to_dev(b, prec))
+            torch.cuda.synchronize()
+        finally:
+            core.set_tuning("row_sweeps", prev)
+        out.append(ud.cpu().numpy())
+    tol = TOL[prec] * (20 if prec == "fp32" else 1)
+    assert rel_err(out[0], ref) < tol
+    assert rel_err(out[1], ref) < tol
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("path", ["box", "march"])
 @pytest.mark.parametrize("k,level", [(1, 3), (2, 3), (3, 2), (3, 4), (4, 3), (3, 5), (5, 2), (6, 2), (7, 2)])
