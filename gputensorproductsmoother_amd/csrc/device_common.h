@@ -66,6 +66,32 @@ namespace gtps
     static constexpr int size = IO + (MH > 0 ? MH * NO : 0);
   };
 
+  // packed DG table offsets (NN = k+1, PD = 2 NN)
+  template <int K>
+  struct DTab
+  {
+    static constexpr int NN = K + 1, PD = 2 * NN;
+    static constexpr int M  = 0;              // cell mass [NN][NN]
+    static constexpr int Lm = M + NN * NN;    // block (c, c-1)
+    static constexpr int Lp = Lm + NN * NN;   // block (c, c+1)
+    static constexpr int Lc = Lp + NN * NN;   // 3 diagonal blocks:
+                                              // interior, first, last cell
+    static constexpr int S   = Lc + 3 * NN * NN;  // 4 patch variants [PD][PD]
+    static constexpr int lam = S + 4 * PD * PD;   // 4 x [PD]
+    static constexpr int E   = lam + 4 * PD;      // child embedding [2][NN][NN]
+    // Off-diagonal blocks in face form: the left neighbour cell w couples to
+    // the patch as e_0 (AR.w) - d0 w(1) / 2 (d0: derivatives of the first
+    // cell's basis at its left end), the right one as e_last (AL.w) + d1 w(0)
+    // / 2.  MS = M S per variant [node][i] (S^T M: nodal -> eigen), EL and ER
+    // the S^T of d0 and d1 on the first and last cell per variant.
+    static constexpr int MS   = E + 2 * NN * NN;
+    static constexpr int EL   = MS + 4 * PD * PD;
+    static constexpr int ER   = EL + 4 * PD;
+    static constexpr int AR   = ER + 4 * PD;
+    static constexpr int AL   = AR + NN;
+    static constexpr int size = AL + NN;
+  };
+
   // Column range of row r of a 2-cell patch matrix (block sparsity: rows
   // inside cell 0 couple to nodes 0..K, rows inside cell 1 to K..2K, the
   // shared vertex row to all).

@@ -35,22 +35,6 @@ namespace gtps
   {
     constexpr int DNT = 256;
 
-    // packed DG table offsets (NN = k+1, PD = 2 NN)
-    template <int K>
-    struct DTab
-    {
-      static constexpr int NN = K + 1, PD = 2 * NN;
-      static constexpr int M  = 0;              // cell mass [NN][NN]
-      static constexpr int Lm = M + NN * NN;    // block (c, c-1)
-      static constexpr int Lp = Lm + NN * NN;   // block (c, c+1)
-      static constexpr int Lc = Lp + NN * NN;   // 3 diagonal blocks:
-                                                // interior, first, last cell
-      static constexpr int S   = Lc + 3 * NN * NN;  // 4 patch variants [PD][PD]
-      static constexpr int lam = S + 4 * PD * PD;   // 4 x [PD]
-      static constexpr int E   = lam + 4 * PD;      // child embedding [2][NN][NN]
-      static constexpr int size = E + 2 * NN * NN;
-    };
-
     __host__ __device__ inline int
     dg_cell_variant(int c, int n)
     {
@@ -1101,6 +1085,29 @@ namespace gtps
           gpu_gen_eig(ctx, PD, L, M, lam, S);
           std::copy(S.begin(), S.end(), tab.begin() + TB::S + v * PD * PD);
           std::copy(lam.begin(), lam.end(), tab.begin() + TB::lam + v * PD);
+          for (int i = 0; i < PD; ++i)
+            {
+              for (int node = 0; node < PD; ++node)
+                {
+                  double s = 0.0;
+                  for (int m = 0; m < PD; ++m)
+                    s += M[node * PD + m] * S[m * PD + i];
+                  tab[TB::MS + (v * PD + node) * PD + i] = s;
+                }
+              double el = 0.0, er = 0.0;
+              for (int a = 0; a < NN; ++a)
+                {
+                  el += d0[a] * S[a * PD + i];
+                  er += d1[a] * S[(NN + a) * PD + i];
+                }
+              tab[TB::EL + v * PD + i] = el;
+              tab[TB::ER + v * PD + i] = er;
+            }
+        }
+      for (int a = 0; a < NN; ++a)
+        {
+          tab[TB::AR + a] = -pf * v1[a] + 0.5 * d1[a];
+          tab[TB::AL + a] = -pf * v0[a] - 0.5 * d0[a];
         }
       // child embedding: fine node q of child c at x = (c + xi_q) / 2
       for (int c = 0; c < 2; ++c)
@@ -1187,6 +1194,13 @@ namespace gtps
                                  first == GTPS_MULT_REV ? 1 : 0, n_sweeps,
                                  (T)lvl->scale, (T)relax, lvl->N);
               GTPS_LAUNCH_CHECK();
+              return;
+            }
+          if (relax == 1.0 && tuning().row_sweeps != 0 &&
+              dg_rows_fit(K, lvl->prec, n))
+            {
+              for (int sw = 0; sw < n_sweeps; ++sw)
+                launch_dg_rows(lvl, u, b, ((first == GTPS_MULT_REV ? 1 : 0) + sw) & 1, nvec);
               return;
             }
           for (int sw = 0; sw < n_sweeps; ++sw)

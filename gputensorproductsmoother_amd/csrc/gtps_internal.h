@@ -306,6 +306,10 @@ namespace gtps
   // operator scratch for batches of nb vectors
   void dg_level_reserve(gtps_dg_level *lvl, int nb);
   bool dg_supported(int k, int prec);
+  // dg_row.hip: one undamped sweep (reverse: colours descending), three
+  // x-colours per launch; the mesh must fit (one row's data in LDS)
+  bool dg_rows_fit(int k, int prec, int n);
+  void launch_dg_rows(const gtps_dg_level *lvl, void *u, const void *b, bool reverse, int nvec);
   // Every DG launcher takes a batch of nb contiguous vectors (stride lvl->N
   // on the level, the coarse level's N for coarse operands); one launch.
   // y = A x (b != NULL: y = b - A x); fused partial dot x.y -> #blocks per

@@ -121,7 +121,9 @@ const char *gtps_version(void);
  *                           small_colour_patches, group_min_patches,
  *                           patches_per_wave, group_waves, row_staged,
  *                           mfma_smoother or mfma_waves: one launch per
- *                           colour with the kernels these knobs choose;
+ *                           colour with the kernels these knobs choose.
+ *                           DG sweeps without damping: 1 three x-colours
+ *                           per launch where a row fits the LDS, 0 one;
  *   "mfma_waves"            matrix-core smoother wavefronts per patch: 4,
  *                           8 (default) or 16.
  * Results do not depend on the knobs beyond round-off.  No reference

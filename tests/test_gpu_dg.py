@@ -118,6 +118,37 @@ def test_dg_smoother_step(core, ctx, k, n, reverse, prec):
     assert rel_err(_host(u), ref) < TOL_SMOOTH[prec]
 
 
+# every remainder of n and n - 1 by 3 (which cells no patch of a class covers)
+ROW_CASES = [(1, 5), (1, 6), (1, 7), (2, 8), (3, 5), (3, 6), (3, 7), (4, 6), (4, 8), (5, 5),
+             (5, 7), (6, 6), (7, 5)]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("reverse", [False, True])
+@pytest.mark.parametrize("k,n", ROW_CASES)
+def test_dg_smoother_rows(core, ctx, k, n, reverse, prec):
+    """Undamped sweeps, three colours per launch (row kernel) and one, agree
+    with the oracle; a non-default penalty goes through the face form."""
+    _skip_unsupported(k, prec)
+    _announce("dg-rows", k, n, "rev" if reverse else "fwd", prec)
+    pf = 1.5 * O.dg_penalty(k)
+    op = core.DGOperator(ctx, 3, k, n, _prec(core, prec), penalty=pf)
+    N = op.n_dofs
+    g = rng(500 + 10 * k + n)
+    b = _round(g.uniform(-1, 1, N), prec)
+    u0 = _round(g.uniform(-1, 1, N), prec)
+    ref = O.dg_smoother_step(3, k, n, b, u0, O.MULT_REV if reverse else O.MULT_FWD, 1.0, pf)
+    for rows in (1, 0):
+        prev = core.set_tuning("row_sweeps", rows)
+        try:
+            u = _dev(u0, _dt(prec))
+            op.smoother_step(u, _dev(b, _dt(prec)), reverse=reverse)
+            got = _host(u)
+        finally:
+            core.set_tuning("row_sweeps", prev)
+        assert rel_err(got, ref) < TOL_SMOOTH[prec]
+
+
 def test_dg_smoother_reduces_error(core, ctx):
     """One symmetric sweep pair contracts the A-norm error of A u = b."""
     _announce("dg-smoother-contract", 3, 6)
