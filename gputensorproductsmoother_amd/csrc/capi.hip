@@ -162,6 +162,14 @@ namespace
     lvl->prec  = precision;
     lvl->tab   = get_tables(ctx, degree);
     lvl->scale = std::pow(std::ldexp(1.0, -level), dim - 2);
+    // without the memory for the intermediate vectors the one-launch
+    // operator runs
+    if (laplace_split_fits(dim, degree, lvl->n, precision) &&
+        hipMalloc(&lvl->split, 2 * lvl->elem() * lvl->N) != hipSuccess)
+      {
+        (void)hipGetLastError();
+        lvl->split = nullptr;
+      }
     return lvl.release();
   }
 

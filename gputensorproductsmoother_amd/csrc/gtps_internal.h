@@ -122,6 +122,9 @@ struct gtps_level
   // operator; both null for the constant-coefficient Laplacian
   void                    *coef  = nullptr;
   void                    *celem = nullptr;
+  // the two intermediate vectors of the two-launch operator
+  // (laplace_split.hip), null where it does not apply
+  void                   *split = nullptr;
   // per vertex patch (lexicographic over (n-1)^3): the separable fit of the
   // variable-coefficient smoother, ratio bins packed as (bx + SEP_HALF) |
   // (by + SEP_HALF) << 8 | (bz + SEP_HALF) << 16, and the scale sigma (level
@@ -134,6 +137,8 @@ struct gtps_level
       (void)hipFree(coef);
     if (celem)
       (void)hipFree(celem);
+    if (split)
+      (void)hipFree(split);
     if (sep_bins)
       (void)hipFree(sep_bins);
     if (sep_sigma)
@@ -281,6 +286,12 @@ namespace gtps
   // first = 0, py = pz = 0)
   void launch_patch_rows(const gtps_level *lvl, void *u, const void *src,
                          int py, int pz, int first, bool zero, double relax);
+
+  // laplace_split.hip: the operator in two launches (needs lvl->split, two
+  // vectors); same contract as launch_laplace
+  bool laplace_split_fits(int dim, int k, int n, int prec);
+  int  launch_laplace_split(const gtps_level *lvl, void *y, const void *x,
+                            const void *b, bool fused_dot);
 
   // coeff.hip: variable-coefficient operator (3D). y = A(c) x (resid:
   // y = b - A(c) x; transpose: y = A(c)^T x); a null level coefficient

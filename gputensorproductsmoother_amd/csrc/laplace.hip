@@ -894,6 +894,12 @@ namespace gtps
   {
     if (lvl->coef)
       return launch_coeff_apply(lvl, y, x, b, fused_dot, false);
+    // two launches where they are faster, unless a knob of the one-launch
+    // kernels was changed
+    const Tuning t, &cur = tuning();
+    if (lvl->split && cur.box_vmult_max_n == t.box_vmult_max_n &&
+        cur.vmult_zdiv == t.vmult_zdiv && cur.vmult_tile == t.vmult_tile)
+      return launch_laplace_split(lvl, y, x, b, fused_dot);
     if (lvl->prec == GTPS_FP32)
       return launch_t<float>(lvl, y, x, b, fused_dot);
     return launch_t<double>(lvl, y, x, b, fused_dot);

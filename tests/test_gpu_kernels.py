@@ -428,3 +428,29 @@ def test_vmult_tiles_k7(core, ctx, level, tile, prec):
     ref = O.laplace_vmult(3, k, level, x)
     assert rel_err(y.cpu().numpy(), ref) < TOL[prec]
     assert rel_err(r.cpu().numpy(), b - ref) < TOL[prec] * 10
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("k,level", [(5, 5), (6, 5), (7, 5), (5, 6)])
+def test_vmult_two_launches(core, ctx, k, level, prec):
+    """The two-launch operator (k >= 5 on 32 cells per direction, k = 5 in
+    FP32 on 64; boundary values in u and b) against the oracle, and the
+    residual written over its right-hand side."""
+    if level == 6 and prec == "fp64":
+        pytest.skip("64 cells: FP32 only")
+    _announce("vmult-two", k, level, prec)
+    g = rng(level * 3 + k)
+    N = n_dofs(3, k, level)
+    x, b = g.uniform(-1, 1, (2, N))
+    if prec == "fp32":
+        x = x.astype(np.float32).astype(np.float64)
+        b = b.astype(np.float32).astype(np.float64)
+    op = core.LaplaceOperator(ctx, 3, k, level, _dt(prec))
+    xd, bd = _to_dev(x, prec), _to_dev(b, prec)
+    y = torch.full_like(xd, float("nan"))
+    op.vmult(y, xd)
+    op.residual(bd, bd, xd)
+    torch.cuda.synchronize()
+    ref = O.laplace_vmult(3, k, level, x)
+    assert rel_err(y.cpu().numpy(), ref) < TOL[prec]
+    assert rel_err(bd.cpu().numpy(), b - ref) < TOL[prec]
