@@ -283,6 +283,15 @@ namespace
           timer->toc_launch(e, ncol);
         return;
       }
+    if (variant == GTPS_ADDITIVE && lvl->dim == 2 && tuning().row_sweeps != 0)
+      {
+        GTPS_REQUIRE(resid != nullptr, "additive sweep needs a residual buffer");
+        const long e = timer ? timer->tic_launch() : -1;
+        launch_additive2d(lvl, u, b, resid, from_zero, relax);
+        if (timer)
+          timer->toc_launch(e, from_zero ? 1 : 2);
+        return;
+      }
     if (from_zero && variant != GTPS_MULT_FWD)
       launch_fill(lvl->ctx->stream, lvl->N, lvl->prec, u, 0.0);
     if (variant == GTPS_ADDITIVE)

@@ -63,7 +63,9 @@ namespace gtps
     static constexpr int at   = mv + NI;
     static constexpr int IE   = at + NI;
     static constexpr int IO   = IE + (MH + 1) * NE;
-    static constexpr int size = IO + (MH > 0 ? MH * NO : 0);
+    // 1/(l_a+l_b) in the even/odd numbering, [b][a]
+    static constexpr int lamInv2p = IO + (MH > 0 ? MH * NO : 0);
+    static constexpr int size     = lamInv2p + NI * NI;
   };
 
   // packed DG table offsets (NN = k+1, PD = 2 NN)

@@ -287,6 +287,12 @@ namespace gtps
   void launch_patch_rows(const gtps_level *lvl, void *u, const void *src,
                          int py, int pz, int first, bool zero, double relax);
 
+  // smoother_add2d.hip: 2D additive smoothing, u += relax sum_P A_P^{-1} r
+  // with r = b - A u formed patch by patch (zero: u = 0 on entry); c is a
+  // level-sized scratch vector
+  void launch_additive2d(const gtps_level *lvl, void *u, const void *b, void *c,
+                         bool zero, double relax);
+
   // laplace_split.hip: the operator in two launches (needs lvl->split, two
   // vectors); same contract as launch_laplace
   bool laplace_split_fits(int dim, int k, int n, int prec);

@@ -373,6 +373,9 @@ namespace gtps
           for (int a = 0; a < NI; ++a)
             tab[TB::lamInv3p + (c * NI + b2) * NI + a] =
               1.0 / (b.lam[perm[c]] + b.lam[perm[b2]] + b.lam[perm[a]]);
+      for (int b2 = 0; b2 < NI; ++b2)
+        for (int a = 0; a < NI; ++a)
+          tab[TB::lamInv2p + b2 * NI + a] = 1.0 / (b.lam[perm[b2]] + b.lam[perm[a]]);
       // face form: S^T M and S^T K applied to the patch nodes
       const int NP    = 2 * K + 1;
       auto      sproj = [&](const std::vector<double> &A, int node, int j) {

@@ -124,6 +124,9 @@ const char *gtps_version(void);
  *                           colour with the kernels these knobs choose.
  *                           DG sweeps without damping: 1 three x-colours
  *                           per launch where a row fits the LDS, 0 one;
+ *                           2D additive sweeps: 1 residual and all patches
+ *                           in one launch, 0 one for the residual and one
+ *                           per colour;
  *   "mfma_waves"            matrix-core smoother wavefronts per patch: 4,
  *                           8 (default) or 16.
  * Results do not depend on the knobs beyond round-off.  No reference

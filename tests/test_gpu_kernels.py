@@ -454,3 +454,34 @@ def test_vmult_two_launches(core, ctx, k, level, prec):
     ref = O.laplace_vmult(3, k, level, x)
     assert rel_err(y.cpu().numpy(), ref) < TOL[prec]
     assert rel_err(bd.cpu().numpy(), b - ref) < TOL[prec]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("zero", [False, True])
+@pytest.mark.parametrize("k,level", [(1, 1), (1, 4), (2, 1), (2, 3), (2, 5), (3, 2), (3, 3),
+                                     (4, 1), (4, 3), (5, 2), (6, 2), (7, 1), (7, 3)])
+def test_additive_2d_one_launch(core, ctx, k, level, zero, prec):
+    """2D additive sweep with residual and patches in one launch (tiles of 8,
+    4 and 2 cells, meshes smaller than a tile) and with one launch per colour,
+    boundary values in u and b, against the oracle."""
+    _announce("additive-2d", k, level, zero, prec)
+    g = rng(level * 13 + k)
+    N = n_dofs(2, k, level)
+    b, u = g.uniform(-1, 1, (2, N))
+    if prec == "fp32":
+        u = u.astype(np.float32).astype(np.float64)
+        b = b.astype(np.float32).astype(np.float64)
+    ref = O.smoother_step(2, k, level, b, np.zeros(N) if zero else u, variant=O.ADDITIVE,
+                          relax=0.4)
+    op = core.LaplaceOperator(ctx, 2, k, level, _dt(prec))
+    sm = core.PatchSmoother(op, core.PatchSmoother.ADDITIVE, 0.4)
+    tol = TOL[prec] * (20 if prec == "fp32" else 1)
+    for one in (1, 0):
+        prev = core.set_tuning("row_sweeps", one)
+        try:
+            ud = _to_dev(u, prec)
+            (sm.vmult if zero else sm.step)(ud, _to_dev(b, prec))
+            torch.cuda.synchronize()
+        finally:
+            core.set_tuning("row_sweeps", prev)
+        assert rel_err(ud.cpu().numpy(), ref) < tol
