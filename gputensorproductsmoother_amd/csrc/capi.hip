@@ -283,7 +283,8 @@ namespace
           timer->toc_launch(e, ncol);
         return;
       }
-    if (variant == GTPS_ADDITIVE && lvl->dim == 2 && tuning().row_sweeps != 0)
+    if (variant == GTPS_ADDITIVE && lvl->dim == 2 && tuning().row_sweeps != 0 &&
+        additive2d_pays(lvl, from_zero))
       {
         GTPS_REQUIRE(resid != nullptr, "additive sweep needs a residual buffer");
         const long e = timer ? timer->tic_launch() : -1;

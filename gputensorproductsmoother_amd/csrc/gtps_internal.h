@@ -290,6 +290,7 @@ namespace gtps
   // smoother_add2d.hip: 2D additive smoothing, u += relax sum_P A_P^{-1} r
   // with r = b - A u formed patch by patch (zero: u = 0 on entry); c is a
   // level-sized scratch vector
+  bool additive2d_pays(const gtps_level *lvl, bool zero);
   void launch_additive2d(const gtps_level *lvl, void *u, const void *b, void *c,
                          bool zero, double relax);
 

@@ -256,6 +256,20 @@ namespace gtps
     }
   } // namespace
 
+  // The tiles recompute the patches and nodes they share, which costs more than
+  // the launches saved once a level fills the GPU.  Measured on MI355X, us per
+  // sweep, this / per colour (from zero): Q2 128^2 FP32 8.6 / 17 (6 / 19),
+  // 512^2 29 / 22 (17 / 27), Q5 128^2 18 / 28 (10 / 31), 512^2 172 / 112
+  // (106 / 124), 1024^2 699 / 383 (414 / 403); FP64 Q2 512^2 33 / 28 (19 /
+  // 35), Q3 512^2 51 / 67 (28 / 80), Q7 512^2 487 / 774 (307 / 797).
+  bool
+  additive2d_pays(const gtps_level *lvl, bool zero)
+  {
+    if (zero)
+      return lvl->N <= 10000000 || lvl->prec == GTPS_FP64;
+    return lvl->N <= 600000 || (lvl->prec == GTPS_FP64 && lvl->k >= 3);
+  }
+
   void
   launch_additive2d(const gtps_level *lvl, void *u, const void *b, void *c, bool zero,
                     double relax)
