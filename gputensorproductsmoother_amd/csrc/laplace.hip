@@ -792,6 +792,17 @@ namespace gtps
                                    : K == 7                ? 256
                                                            : 2048;
             int zc = (int)(((long long)n * tx * ty + zdiv - 1) / zdiv);
+            // FP32: a chunk re-reads 2k+1 planes, mostly from the caches, while
+            // chunks of more than 3 cells leave too few work-groups to hide
+            // the plane chain (k = 3 and FP64 gain nothing: more registers,
+            // fewer resident work-groups).  Measured on MI355X, us (vmult,
+            // residual), capped / not: Q1 256^3 54 / 78, 68 / 110, Q2 128^3
+            // 54 / 72, 67 / 94, Q4 64^3 102 / 141, 139 / 206
+            if (sizeof(T) == 4 && (K <= 2 || K == 4) && tuning().vmult_zdiv == 0)
+              zc = std::min(zc, 3);
+            if (fused_dot)  // one partial per work-group
+              zc = std::max(zc, (int)(((long long)n * tx * ty + lvl->ctx->ws.capacity - 1) /
+                                      std::max(1, lvl->ctx->ws.capacity - tx * ty)));
             zc     = std::max(1, std::min(zc, n));
             const int tz = (n + zc - 1) / zc;
             const dim3 grid(tx, ty, tz);
