@@ -124,6 +124,113 @@ namespace gtps
     }
 
     // ------------------------------------------------------------------
+    // Restriction along one direction, one coarse cell's K nodes per thread
+    // (the cell's fine nodes and, for the vertex, those of the cell before).
+    // restrict_line_kernel: any direction but x, lanes along the contiguous
+    // inner extent (blockIdx.y = coarse cell, blockIdx.z = outer index), the
+    // embedding as uniform loads.  restrict_row_kernel: along x, rows
+    // staged in LDS (rr of them).  With the passes in the order z, y, x the strided
+    // direction works on a quarter of the data.  One thread per coarse node
+    // with generic indices, x first, took 106 us at Q7 32^3 FP32 and 195 us in
+    // FP64; this takes 47 and 68 (Q5 35 and 62: 18 and 27).
+    template <int K, typename T>
+    __device__ __forceinline__ void
+    restrict_cell(const T *__restrict__ E, const T (&own)[2 * K], const T (&prev)[2 * K - 1],
+                  T (&o)[K])
+    {
+      constexpr int N = K + 1;
+      T             v = own[0];
+#pragma unroll
+      for (int q = 1; q < 2 * K; ++q)
+        v += E[q * N] * own[q];
+#pragma unroll
+      for (int q = 1; q < 2 * K; ++q)
+        v += E[q * N + K] * prev[q - 1];
+      o[0] = v;
+#pragma unroll
+      for (int a = 1; a < K; ++a)
+        {
+          T w = 0;
+#pragma unroll
+          for (int q = 1; q < 2 * K; ++q)
+            w += E[q * N + a] * own[q];
+          o[a] = w;
+        }
+    }
+
+    template <int K, typename T>
+    __global__ void __launch_bounds__(TR_NT)
+    restrict_line_kernel(const T *__restrict__ in, T *__restrict__ out,
+                         const T *__restrict__ tab, const long long inner, const int nc)
+    {
+      const long long i = (long long)blockIdx.x * TR_NT + threadIdx.x;
+      if (i >= inner)
+        return;
+      const int cc = blockIdx.y;
+      const T  *f  = in + i + ((long long)blockIdx.z * (2 * K * nc + 1) + 2 * K * cc) * inner;
+      T        *c  = out + i + ((long long)blockIdx.z * (K * nc + 1) + K * cc) * inner;
+      T         own[2 * K], prev[2 * K - 1], o[K];
+      own[0] = f[0];
+#pragma unroll
+      for (int q = 1; q < 2 * K; ++q)
+        own[q] = cc < nc ? f[q * inner] : T(0);
+#pragma unroll
+      for (int q = 1; q < 2 * K; ++q)
+        prev[q - 1] = cc > 0 ? f[(q - 2 * K) * inner] : T(0);
+      restrict_cell<K>(tab + Tab<K>::E, own, prev, o);
+      c[0] = o[0];
+      if (cc < nc)
+        {
+#pragma unroll
+          for (int a = 1; a < K; ++a)
+            c[a * inner] = o[a];
+        }
+    }
+
+    // last pass: rr rows (y, z) of the coarse mesh; ADD or store, interior only
+    template <int K, typename T, bool ADD>
+    __global__ void __launch_bounds__(TR_NT)
+    restrict_row_kernel(const T *__restrict__ in, T *__restrict__ out,
+                        const T *__restrict__ tab, const int dim, const int nc,
+                        const int Nc1, const long long rows, const int rr)
+    {
+      extern __shared__ double smem_raw[];
+      T              *sm  = reinterpret_cast<T *>(smem_raw);
+      const int       Nf1 = 2 * K * nc + 1;
+      const long long r0  = (long long)blockIdx.x * rr;
+      const int       nr  = rows - r0 < rr ? (int)(rows - r0) : rr;
+      for (int i = threadIdx.x; i < nr * Nf1; i += TR_NT)
+        sm[i] = in[r0 * Nf1 + i];
+      __syncthreads();
+      for (int t = threadIdx.x; t < nr * nc; t += TR_NT)
+        {
+          const int       r = t / nc, cc = t - r * nc;
+          const long long row = r0 + r, z = row / Nc1, y = row - z * Nc1;
+          if (y == 0 || y == Nc1 - 1 || (dim == 3 && (z == 0 || z == Nc1 - 1)))
+            continue;
+          const T *f = sm + r * Nf1 + 2 * K * cc;
+          T       *c = out + row * Nc1 + K * cc;
+          T        own[2 * K], prev[2 * K - 1], o[K];
+#pragma unroll
+          for (int q = 0; q < 2 * K; ++q)
+            own[q] = f[q];
+#pragma unroll
+          for (int q = 1; q < 2 * K; ++q)
+            prev[q - 1] = cc > 0 ? f[q - 2 * K] : T(0);
+          restrict_cell<K>(tab + Tab<K>::E, own, prev, o);
+#pragma unroll
+          for (int a = 0; a < K; ++a)
+            if (a > 0 || cc > 0)
+              {
+                if (ADD)
+                  c[a] += o[a];
+                else
+                  c[a] = o[a];
+              }
+        }
+    }
+
+    // ------------------------------------------------------------------
     // Fused 3D kernels: one work-group owns a tile of CX x CY x CZ coarse
     // cells.  Prolongation stages the coarse tile (k C + 1 nodes per
     // direction, Dirichlet nodes as zero) in LDS, applies E along x, y, z in
@@ -475,7 +582,7 @@ namespace gtps
           return;
         }
       // the restriction window outgrows 64 KiB of LDS beyond k = 4: those
-      // degrees keep the three separable passes below
+      // degrees take three separable passes below
       if constexpr (K <= 4)
         if (dim == 3)
           {
@@ -491,6 +598,12 @@ namespace gtps
             GTPS_LAUNCH_CHECK();
             return;
           }
+      // rows per work-group of the restriction's last pass: several once
+      // there are work-groups enough (2D Q2 1024^2 restriction: 37 us with 128
+      // of 8 rows, 15 us with one row each)
+      const long long rows = dim == 3 ? (long long)Nc1 * Nc1 : Nc1;
+      const int       rr   = (int)std::max<long long>(1, std::min<long long>(8, rows / 2048));
+      const size_t    lds  = (size_t)rr * Nf1 * sizeof(T);
       if (prolong)
         {
           int e0[3] = {Nc1, Nc1, dim == 3 ? Nc1 : 1};
@@ -506,8 +619,42 @@ namespace gtps
               pass<K, T, true, false, 1>(s, t2, fine, tab, dim, 2, e2, e3, nc, Nc1);
             }
         }
+      else if (nc < 65535 && Nc1 < 65535 && lds <= 160 * 1024)
+        {
+          auto line = [&](const T *in, T *out, long long inner, int outer) {
+            hipLaunchKernelGGL((restrict_line_kernel<K, T>),
+                               dim3((unsigned)((inner + TR_NT - 1) / TR_NT), nc + 1, outer),
+                               dim3(TR_NT), 0, s, in, out, tab, inner, nc);
+            GTPS_LAUNCH_CHECK();
+          };
+          const T *last;
+          if (dim == 2)
+            {
+              line(fine_in, t1, Nf1, 1);
+              last = t1;
+            }
+          else
+            {
+              line(fine_in, t1, (long long)Nf1 * Nf1, 1);
+              line(t1, t2, Nf1, Nc1);
+              last = t2;
+            }
+          auto            row  = [&](auto kern) {
+            if (lds > 65536)
+              GTPS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            hipLaunchKernelGGL(kern, dim3((unsigned)((rows + rr - 1) / rr)), dim3(TR_NT), lds, s,
+                               last, coarse, tab, dim, nc, Nc1, rows, rr);
+            GTPS_LAUNCH_CHECK();
+          };
+          if (store)
+            row(restrict_row_kernel<K, T, false>);
+          else
+            row(restrict_row_kernel<K, T, true>);
+        }
       else
         {
+          // rows beyond the LDS or the grid: one thread per coarse node
           int e0[3] = {Nf1, Nf1, dim == 3 ? Nf1 : 1};
           int e1[3] = {Nc1, Nf1, dim == 3 ? Nf1 : 1};
           int e2[3] = {Nc1, Nc1, dim == 3 ? Nf1 : 1};

@@ -485,3 +485,25 @@ def test_additive_2d_one_launch(core, ctx, k, level, zero, prec):
         finally:
             core.set_tuning("row_sweeps", prev)
         assert rel_err(ud.cpu().numpy(), ref) < tol
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("dim,k,level", [(3, 5, 5), (3, 6, 3), (3, 7, 4), (2, 1, 8), (2, 3, 6),
+                                         (2, 7, 5)])
+def test_restriction_line_passes(core, ctx, dim, k, level, prec):
+    """Restriction in line passes (3D from degree 5 on, 2D; one and several
+    rows per work-group in the last pass) against the oracle, adding to
+    coarse values that are kept on the Dirichlet nodes."""
+    _announce("restrict-lines", dim, k, level, prec)
+    g = rng(level * 17 + k)
+    fine = g.uniform(-1, 1, n_dofs(dim, k, level))
+    coarse = g.uniform(-1, 1, n_dofs(dim, k, level - 1))
+    if prec == "fp32":
+        fine = fine.astype(np.float32).astype(np.float64)
+        coarse = coarse.astype(np.float32).astype(np.float64)
+    ref = O.restrict_add(dim, k, level, fine, coarse)
+    tr = core.MGTransferCUDA(ctx, dim, k, 1, level, _dt(prec))
+    cd = _to_dev(coarse, prec)
+    tr.restrict_and_add(level, cd, _to_dev(fine, prec))
+    torch.cuda.synchronize()
+    assert rel_err(cd.cpu().numpy(), ref) < TOL[prec]
