@@ -362,12 +362,14 @@ struct gtps_mg : LaunchTimer
 
   // the per-iteration preconditioning sequence (V-cycle, r.z, beta,
   // deferred x update, p update) replayed as one HIP graph; captured lazily
-  // on a private stream, again when the solution vector changes
+  // on a private stream. Its last kernel finds the solution vector through
+  // xslot (device), which every solve sets by a launch of its own: a capture
+  // costs 0.2 ms and more, and a solution vector is new for most solves
   bool                       use_graph  = true;
   hipStream_t                cap_stream = nullptr;
   hipGraphExec_t             dir_exec   = nullptr;
   unsigned long long         dir_gen    = 0;  // tuning generation at capture
-  double                    *dir_x      = nullptr;  // solution at capture
+  double                   **xslot      = nullptr;
 
   // the V-cycle from level 2 down as a dense matrix (coarse.hip), built
   // on first use and dropped when the operators change
@@ -512,7 +514,7 @@ struct gtps_mg : LaunchTimer
   // beta p; every other buffer is owned by the hierarchy, so the sequence
   // can be captured
   void
-  enqueue_direction(double *x)
+  enqueue_direction()
   {
     hipStream_t     s   = ctx->stream;
     double         *sc  = ctx->ws.scalars;
@@ -529,16 +531,15 @@ struct gtps_mg : LaunchTimer
     toc(GTPS_PROF_VCYCLE, e);
     const int nb = launch_dot_partials(s, N, r, z64, z32, pt, ctx->ws.capacity);
     launch_finalize_op(s, pt, nb, sc, cg::RZ, cg::OP_SHIFT_BETA);
-    launch_cg_update_p(s, N, p, z64, z32, sc, x);
+    launch_cg_update_p(s, N, p, z64, z32, sc, xslot);
   }
 
   // a graph captured before the last gtps_set_tuning may replay other
-  // kernels than an eager launch would, and one captured for another
-  // solution vector writes there: capture it again
+  // kernels than an eager launch would: capture it again
   void
-  drop_stale_graph(const double *x)
+  drop_stale_graph()
   {
-    if (dir_exec && (dir_gen != tuning().generation || dir_x != x))
+    if (dir_exec && dir_gen != tuning().generation)
       {
         GTPS_HIP(hipStreamSynchronize(ctx->stream));
         (void)hipGraphExecDestroy(dir_exec);
@@ -546,8 +547,21 @@ struct gtps_mg : LaunchTimer
       }
   }
 
+  // a graph captured with a coefficient in place on every level holds for
+  // the next coefficient too: the values change, the buffers do not
+  bool
+  coefficient_in_place() const
+  {
+    if (coef64.empty())
+      return false;
+    for (int l = 1; l <= maxl; ++l)
+      if (!lv[l]->coef || !lv[l]->sep_bins || !lv[l]->sep_sigma)
+        return false;
+    return true;
+  }
+
   void
-  capture_direction(double *x)
+  capture_direction()
   {
     if (!cap_stream)
       GTPS_HIP(hipStreamCreateWithFlags(&cap_stream, hipStreamNonBlocking));
@@ -558,7 +572,7 @@ struct gtps_mg : LaunchTimer
       {
         GTPS_HIP(hipStreamBeginCapture(cap_stream,
                                        hipStreamCaptureModeThreadLocal));
-        enqueue_direction(x);
+        enqueue_direction();
         GTPS_HIP(hipStreamEndCapture(cap_stream, &graph));
       }
     catch (...)
@@ -580,23 +594,22 @@ struct gtps_mg : LaunchTimer
     (void)hipGraphDestroy(graph);
     GTPS_HIP(e);
     dir_gen = tuning().generation;
-    dir_x   = x;
   }
 
-  // x: the solution, which receives the deferred x += alpha p
+  // the solution named in xslot receives the deferred x += alpha p
   void
-  direction(double *x)
+  direction()
   {
     ensure_dense();
     // stage timers need eager launches
     if (!use_graph || prof_mask != 0)
       {
-        enqueue_direction(x);
+        enqueue_direction();
         return;
       }
-    drop_stale_graph(x);
+    drop_stale_graph();
     if (!dir_exec)
-      capture_direction(x);
+      capture_direction();
     GTPS_HIP(hipGraphLaunch(dir_exec, ctx->stream));
   }
 
@@ -815,6 +828,7 @@ struct gtps_mg : LaunchTimer
     dfree(r);
     dfree(p);
     dfree(q);
+    dfree(xslot);
     if (ev)
       (void)hipEventDestroy(ev);
     for (hipEvent_t e : ev_pool)
@@ -1836,6 +1850,7 @@ extern "C"
       mg->r             = (double *)dmalloc(sizeof(double) * N);
       mg->p             = (double *)dmalloc(sizeof(double) * N);
       mg->q             = (double *)dmalloc(sizeof(double) * N);
+      mg->xslot         = (double **)dmalloc(sizeof(double *));
       GTPS_HIP(hipEventCreateWithFlags(&mg->ev, hipEventDisableTiming));
       // zero boundary entries of the level vectors once: kernels never write
       // them except through vmult / residual
@@ -2088,9 +2103,9 @@ extern "C"
       GTPS_REQUIRE(mg, "NULL argument");
       set_device(mg->ctx);
       hipStream_t s = mg->ctx->stream;
-      // kernels change: the captured preconditioning graph is stale
       GTPS_HIP(hipStreamSynchronize(s));
-      if (mg->dir_exec)
+      // kernels or buffers change: the captured preconditioning graph is stale
+      if (mg->dir_exec && !(coef && mg->coefficient_in_place()))
         {
           (void)hipGraphExecDestroy(mg->dir_exec);
           mg->dir_exec = nullptr;
@@ -2221,7 +2236,10 @@ extern "C"
       // r0 (a zero or non-finite r0 discards it; alpha = 0 here, so its x
       // update leaves x as it is)
       if (maxit > 0)
-        mg->direction(x);
+        {
+          launch_set_pointer(s, mg->xslot, x);
+          mg->direction();
+        }
       const double r0 = wait_rr();
       if (history)
         history[0] = r0;
@@ -2261,7 +2279,7 @@ extern "C"
             speculate = rn * (rn / rn_prev) > 0.25 * rtol * r0;
           if (speculate)
             {
-              mg->direction(x);
+              mg->direction();
               x_pending = false;
             }
           rn_prev = rn;
@@ -2280,7 +2298,7 @@ extern "C"
             }
           if (!speculate && it_done < maxit)
             {
-              mg->direction(x);
+              mg->direction();
               x_pending = false;
             }
         }

@@ -447,10 +447,12 @@ namespace gtps
                            const double *scalars, double *partials,
                            int capacity);
   // x == nullptr in launch_cg_update_xr defers x += alpha p to the next
-  // launch_cg_update_p with x (or to launch_cg_add_alpha_p)
+  // launch_cg_update_p with x (or to launch_cg_add_alpha_p). There x is read
+  // from a device slot, so that a captured launch serves every solution vector
   void launch_cg_update_p(hipStream_t s, long long n, double *p,
                           const double *z, const float *z32,
-                          const double *scalars, double *x = nullptr);
+                          const double *scalars, double *const *xslot = nullptr);
+  void launch_set_pointer(hipStream_t s, double **slot, double *x);
   void launch_cg_add_alpha_p(hipStream_t s, long long n, double *x,
                              const double *p, const double *scalars);
 

@@ -272,9 +272,10 @@ namespace gtps
     cg_update_p_kernel(long long n, double *__restrict__ p,
                        const double *__restrict__ z,
                        const float *__restrict__ z32,
-                       const double *__restrict__ sc, double *__restrict__ x)
+                       const double *__restrict__ sc, double *const *__restrict__ xslot)
     {
       const double beta = sc[cg::BETA], alpha = sc[cg::ALPHA];
+      double *__restrict__ x = xslot ? *xslot : nullptr;
       for (long long i = (long long)blockIdx.x * VNT + threadIdx.x; i < n;
            i += (long long)gridDim.x * VNT)
         {
@@ -284,6 +285,12 @@ namespace gtps
             x[i] += alpha * pi;
           p[i] = zi + beta * pi;
         }
+    }
+
+    __global__ void
+    set_pointer_kernel(double **slot, double *x)
+    {
+      *slot = x;
     }
 
     // x += alpha p: the deferred update of the last step
@@ -475,10 +482,17 @@ namespace gtps
 
   void
   launch_cg_update_p(hipStream_t s, long long n, double *p, const double *z,
-                     const float *z32, const double *scalars, double *x)
+                     const float *z32, const double *scalars, double *const *xslot)
   {
     hipLaunchKernelGGL(cg_update_p_kernel, dim3(grid_for(n)), dim3(VNT), 0, s,
-                       n, p, z, z32, scalars, x);
+                       n, p, z, z32, scalars, xslot);
+    GTPS_LAUNCH_CHECK();
+  }
+
+  void
+  launch_set_pointer(hipStream_t s, double **slot, double *x)
+  {
+    hipLaunchKernelGGL(set_pointer_kernel, dim3(1), dim3(1), 0, s, slot, x);
     GTPS_LAUNCH_CHECK();
   }
 

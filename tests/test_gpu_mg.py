@@ -163,6 +163,31 @@ def test_graph_replays_match_eager(core, ctx, prec):
         assert torch.equal(x_g, x_e), rep
 
 
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_graph_across_solutions_and_coefficients(core, ctx, prec):
+    """One hierarchy solves into new solution vectors (all kept alive) and
+    under changing coefficients, none included; every solve has bitwise the
+    iterates of a hierarchy without a graph, and leaves the solutions of the
+    solves before it alone."""
+    _announce("graph-new-x", prec)
+    dim, k, level = 3, 2, 3
+    dt = torch.float32 if prec == "fp32" else torch.float64
+    coefs = [None, None] + [torch.tensor(np.exp(0.5 * rng(40 + i).standard_normal(
+        (1 << level) ** 3)), device="cuda:0") for i in range(2)] + [None]
+    mg_e, mg_g = (core.MultigridSolvers(ctx, dim, k, level, dt) for _ in range(2))
+    mg_e.set_graph(False)
+    got, want = [], []
+    for i, c in enumerate(coefs * 2):
+        b = torch.tensor(O.rhs_random(dim, k, level) * (1.0 + i), device="cuda:0")
+        for m, out in ((mg_e, want), (mg_g, got)):
+            m.set_coefficient(c)
+            out.append(m.solve_cg(b, rtol=1e-8)[0])
+    torch.cuda.synchronize()
+    for i, (x, y) in enumerate(zip(got, want)):
+        assert torch.equal(x, y), i
+    assert len({x.data_ptr() for x in got}) == len(got)
+
+
 # ------------------------------------------------------------ full multigrid
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("dim,k,level,n_cycles,coef", [
