@@ -740,7 +740,7 @@ def main():
     ap.add_argument("--traffic-summary", nargs=2, metavar=("FETCH_DIR", "WRITE_DIR"),
                     help="write profiles/traffic.json from two rocprofv3 --pmc runs of "
                          "--kernels (no GPU work)")
-    ap.add_argument("--traffic-kernel", default="patch3d_group_kernel<3, float, 0, 2, 4>")
+    ap.add_argument("--traffic-kernel", default="patch_rows3d_kernel<3, float, false, 16, 256>")
     ap.add_argument("--traffic-out", default=os.path.join(ROOT, "profiles", "traffic.json"),
                     help="output of --traffic-summary")
     ap.add_argument("--solve-trace", metavar="c2|c3|c4|c5",

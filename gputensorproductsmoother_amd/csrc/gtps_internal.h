@@ -204,7 +204,10 @@ namespace gtps
   // process-wide tuning knobs (gtps_set_tuning)
   struct Tuning
   {
-    // smoother colours with at most this many patches use the single-patch
+    // The knobs up to mfma_waves choose among the kernels of one colour:
+    // 3D additive smoothing, a lone patch of degree 6 or 7 in FP32, and
+    // 3D multiplicative sweeps once one of them is changed (row_sweeps).
+    // Smoother colours with at most this many patches use the single-patch
     // kernel, larger ones the multi-patch kernel (k <= 3).  Measured on
     // MI355X at 64^3 Q3 the single-patch kernel is at least as fast on every
     // level (4.3-7.7 us per coarse-level launch instead of 11-13 us; level 6

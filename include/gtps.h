@@ -110,10 +110,12 @@ const char *gtps_version(void);
  *                           256, 3 (default): 0 in FP32, 1 in FP64; for
  *                           k = 7: 0: 8x2 cells and 512 threads, 1: 4x4
  *                           and 1024, 2 and 3 (default): 4x4 and 512;
- *   "mfma_smoother"         1 (default): 3D FP32 multiplicative smoothing of
- *                           degree 4..7 runs its 1D contractions on the
- *                           matrix cores (v_mfma_f32_16x16x4f32, patches
- *                           padded to 16^3); 0: the LDS/FMA kernel.
+ *   "mfma_smoother"         where a sweep launches colour by colour (see
+ *                           row_sweeps), 1 (default): 3D FP32
+ *                           multiplicative smoothing of degree 4..7 runs
+ *                           its 1D contractions on the matrix cores
+ *                           (v_mfma_f32_16x16x4f32, patches padded to
+ *                           16^3); 0: the LDS/FMA kernel.
  *   "row_sweeps"            1 (default): 3D multiplicative sweeps smooth the
  *                           two colours of equal y and z parity in one
  *                           launch, one work-group per x-row of patches;
@@ -326,8 +328,9 @@ int gtps_mg_coefficient_gradient(gtps_mg *mg, double *grad,
                                  const double *lambda, const double *u);
 
 /* Replay the per-iteration preconditioning sequence (V-cycle, r.z, beta,
- * p update; about 130 kernels for 6 levels) as one HIP graph captured on the
- * first solve (enable != 0, the default), or launch it kernel by kernel.
+ * p update; several dozen kernels for 6 levels) as one HIP graph captured on
+ * the first solve (enable != 0, the default) and kept for other solutions,
+ * right-hand sides and coefficients, or launch it kernel by kernel.
  * The graph uses no memset nodes.  Stage timers force kernel-by-kernel
  * launches.  No reference counterpart (the reference launches every kernel
  * on the default stream and synchronises after each stage,
