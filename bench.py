@@ -182,8 +182,8 @@ def config_report(args):
             b = torch.tensor(problems.rhs_constant(dim, k, level, cell_mass(k)), device=dev)
             r = solve_pair(dim, k, level, b, 1e-8)
             line = {"config": "C3", "workload": "3D Q7 Poisson f=1, 32^3 cells, "
-                    "multiplicative smoother (FP32: 1D contractions on the matrix cores; "
-                    "FP64: LDS/FMA kernel), CG to 1e-8", "n_dofs": b.numel(),
+                    "multiplicative smoother, "
+                    "CG to 1e-8", "n_dofs": b.numel(),
                     "mfma_utilisation": mfma_report(core, ctx, k, level, reps),
                     "hbm_per_kernel": hbm_report(core, ctx, k, level, reps), **r}
         elif name == "c4":
