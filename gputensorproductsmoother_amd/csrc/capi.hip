@@ -567,6 +567,7 @@ struct gtps_mg : LaunchTimer
       GTPS_HIP(hipStreamCreateWithFlags(&cap_stream, hipStreamNonBlocking));
     hipStream_t saved = ctx->stream;
     ctx->stream       = cap_stream;
+    ctx->own_capture  = true;
     hipGraph_t graph  = nullptr;
     try
       {
@@ -577,7 +578,8 @@ struct gtps_mg : LaunchTimer
       }
     catch (...)
       {
-        ctx->stream = saved;
+        ctx->stream      = saved;
+        ctx->own_capture = false;
         if (!graph)
           {
             hipGraph_t g = nullptr;
@@ -589,7 +591,8 @@ struct gtps_mg : LaunchTimer
           (void)hipGraphDestroy(graph);
         throw;
       }
-    ctx->stream = saved;
+    ctx->stream      = saved;
+    ctx->own_capture = false;
     hipError_t e = hipGraphInstantiate(&dir_exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     GTPS_HIP(e);

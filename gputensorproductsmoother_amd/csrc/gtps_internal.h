@@ -105,6 +105,9 @@ struct gtps_ctx
   int                                                     device = 0;
   hipStream_t                                             stream = nullptr;
   bool                                                    own_stream = false;
+  // a hierarchy is recording its own graph, which it replays on `stream` only
+  // and destroys before its levels
+  bool                                                    own_capture = false;
   gtps::Workspace                                         ws;
   std::map<int, std::unique_ptr<gtps::DegreeTables>>      tables;
 };
@@ -123,7 +126,8 @@ struct gtps_level
   void                    *coef  = nullptr;
   void                    *celem = nullptr;
   // the two intermediate vectors of the two-launch operator
-  // (laplace_split.hip), null where it does not apply
+  // (laplace_split.hip), null where it does not apply. A caller's graph never
+  // holds them: it may outlive the level, and several may run at once
   void                   *split = nullptr;
   // per vertex patch (lexicographic over (n-1)^3): the separable fit of the
   // variable-coefficient smoother, ratio bins packed as (bx + SEP_HALF) |

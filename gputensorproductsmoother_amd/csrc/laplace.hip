@@ -897,6 +897,22 @@ namespace gtps
           default: throw Error(GTPS_EINVAL, "degree must be in 1..7");
         }
     }
+
+    // the context's stream records a graph that its caller will replay when
+    // and where it likes
+    bool
+    callers_capture(const gtps_ctx *ctx)
+    {
+      if (ctx->own_capture)
+        return false;
+      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess)
+        {
+          (void)hipGetLastError();
+          return true;
+        }
+      return st != hipStreamCaptureStatusNone;
+    }
   } // namespace
 
   int
@@ -906,10 +922,12 @@ namespace gtps
     if (lvl->coef)
       return launch_coeff_apply(lvl, y, x, b, fused_dot, false);
     // two launches where they are faster, unless a knob of the one-launch
-    // kernels was changed
+    // kernels was changed or the launch would bind the level's scratch into a
+    // caller's graph
     const Tuning t, &cur = tuning();
     if (lvl->split && cur.box_vmult_max_n == t.box_vmult_max_n &&
-        cur.vmult_zdiv == t.vmult_zdiv && cur.vmult_tile == t.vmult_tile)
+        cur.vmult_zdiv == t.vmult_zdiv && cur.vmult_tile == t.vmult_tile &&
+        !callers_capture(lvl->ctx))
       return launch_laplace_split(lvl, y, x, b, fused_dot);
     if (lvl->prec == GTPS_FP32)
       return launch_t<float>(lvl, y, x, b, fused_dot);

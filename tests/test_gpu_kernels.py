@@ -457,6 +457,46 @@ def test_vmult_two_launches(core, ctx, k, level, prec):
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_vmult_captured_by_caller(core, prec):
+    """Two graphs that a program records from one operator hold no scratch of
+    its level: they replay on two streams at once and after the operator is
+    gone, bitwise equal to the one-launch operator."""
+    _announce("vmult-captured", prec)
+    k, level = 5, 5
+    N = n_dofs(3, k, level)
+    st = [torch.cuda.Stream() for _ in range(2)]
+    cx = core.Context(0, st[0].cuda_stream)
+    op = core.LaplaceOperator(cx, 3, k, level, _dt(prec))
+    x = [_to_dev(rng(70 + i).uniform(-1, 1, N), prec) for i in range(2)]
+    y = [torch.empty_like(v) for v in x]
+    want = [torch.empty_like(v) for v in x]
+    torch.cuda.synchronize()
+    prev = core.set_tuning("box_vmult_max_n", 15)  # any change: one launch
+    try:
+        for v, w in zip(x, want):
+            op.vmult(w, v)
+    finally:
+        core.set_tuning("box_vmult_max_n", prev)
+    torch.cuda.synchronize()
+    graphs = []
+    for v, w in zip(x, y):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st[0]):
+            op.vmult(w, v)
+        graphs.append(g)
+    del op
+    for rep in range(3):
+        for w in y:
+            w.zero_()
+        torch.cuda.synchronize()
+        for s, g in zip(st, graphs):
+            with torch.cuda.stream(s):
+                g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(y, want)), rep
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("zero", [False, True])
 @pytest.mark.parametrize("k,level", [(1, 1), (1, 4), (2, 1), (2, 3), (2, 5), (3, 2), (3, 3),
                                      (4, 1), (4, 3), (5, 2), (6, 2), (7, 1), (7, 3)])
