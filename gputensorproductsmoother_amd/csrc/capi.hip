@@ -146,6 +146,19 @@ namespace
     GTPS_REQUIRE(level <= (dim == 3 ? 12 : 20), "level too large");
   }
 
+  // the intermediate vectors of the two-launch operator; without the memory
+  // for them the one-launch operator runs
+  void
+  alloc_split(gtps_level *lvl)
+  {
+    if (laplace_split_fits(lvl->dim, lvl->k, lvl->n, lvl->prec) &&
+        hipMalloc(&lvl->split, 2 * lvl->elem() * lvl->N) != hipSuccess)
+      {
+        (void)hipGetLastError();
+        lvl->split = nullptr;
+      }
+  }
+
   gtps_level *
   make_level(gtps_ctx *ctx, int dim, int degree, int level, int precision)
   {
@@ -162,14 +175,7 @@ namespace
     lvl->prec  = precision;
     lvl->tab   = get_tables(ctx, degree);
     lvl->scale = std::pow(std::ldexp(1.0, -level), dim - 2);
-    // without the memory for the intermediate vectors the one-launch
-    // operator runs
-    if (laplace_split_fits(dim, degree, lvl->n, precision) &&
-        hipMalloc(&lvl->split, 2 * lvl->elem() * lvl->N) != hipSuccess)
-      {
-        (void)hipGetLastError();
-        lvl->split = nullptr;
-      }
+    alloc_split(lvl.get());
     return lvl.release();
   }
 
@@ -190,6 +196,14 @@ namespace
   {
     GTPS_REQUIRE(lvl->dim == 3, "the variable-coefficient operator is 3D");
     const long long ncells = (long long)lvl->n * lvl->n * lvl->n;
+    if (lvl->split)
+      {
+        // only the constant-coefficient operator uses it (a graph of the
+        // hierarchy that does was dropped by the caller)
+        GTPS_HIP(hipStreamSynchronize(lvl->ctx->stream));
+        dfree(lvl->split);
+        lvl->split = nullptr;
+      }
     if (!lvl->coef)
       lvl->coef = dmalloc(lvl->elem() * ncells);
     ensure_celem(lvl);
@@ -227,6 +241,7 @@ namespace
         dfree(lvl->sep_sigma);
         lvl->sep_bins  = nullptr;
         lvl->sep_sigma = nullptr;
+        alloc_split(lvl);
       }
   }
 

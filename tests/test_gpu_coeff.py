@@ -260,3 +260,36 @@ def test_autograd_boundary_gradient_of_b(core, ctx):
     lam = np.linalg.solve(A.T, w.cpu().numpy())
     assert rel_err(b.grad.cpu().numpy(), lam) < 1e-9
     assert np.abs(b.grad.cpu().numpy()[bm]).max() > 0
+
+
+def test_coefficient_releases_two_launch_scratch(core, ctx):
+    """While a coefficient is set the level does not hold the two vectors of
+    the constant-coefficient operator, and clearing it brings back the same
+    operator (bitwise)."""
+    k, level = 5, 5
+    _announce("coeff-split", k, level)
+    N = n_dofs(3, k, level)
+    c = _dev(_coef(level))
+    x = _dev(rng(46).uniform(-1, 1, N), torch.float32)
+    first, op = (core.LaplaceOperator(ctx, 3, k, level, torch.float32) for _ in range(2))
+    first.set_coefficient(c)  # the degree's tables are the context's
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    op.vmult(y, x)
+    op.vmult_transpose(z, x)  # the element vectors of the cell-wise operator
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    op.set_coefficient(c)
+    ctx.synchronize()
+    # 33 MB less, some 0.4 MB of coefficient data more
+    assert torch.cuda.mem_get_info()[0] - before > 1.8 * 4 * N
+    op.set_coefficient(None)
+    op.vmult(z, x)
+    torch.cuda.synchronize()
+    assert torch.equal(y, z)
+    prev = core.set_tuning("box_vmult_max_n", 15)  # one launch
+    try:
+        op.vmult(y, x)
+    finally:
+        core.set_tuning("box_vmult_max_n", prev)
+    torch.cuda.synchronize()
+    assert not torch.equal(y, z)
