@@ -267,6 +267,21 @@ namespace
            c.mfma_waves == t.mfma_waves;
   }
 
+  // Whether two colours per launch are the faster form of a sweep (zero: it
+  // starts from u = 0 itself; a reverse sweep is filled first).  A single
+  // patch has one colour, so nothing is shared and the shorter kernel wins.
+  // Measured on MI355X in a graph, us per sweep, row / per colour: one patch
+  // onto u Q1 3.0 / 2.2, Q3 4.4 / 3.2 (FP64 5.3 / 3.7), Q4 5.5 / 6.3 (FP64
+  // 6.7 / 8.6), Q7 FP64 19.3 / 24.0, and against the matrix cores in FP32 Q5
+  // 7.4 / 7.2, Q6 9.8 / 7.3, Q7 12.3 / 7.8; from zero Q1 2.5 / 2.1, Q3 3.4 /
+  // 3.0 (FP64 3.8 / 3.2), Q4 4.1 / 8.1, Q5 5.8 / 9.0, Q7 8.1 / 9.7.
+  bool
+  rows_pay(const gtps_level *lvl, bool zero)
+  {
+    const bool f32 = lvl->prec == GTPS_FP32;
+    return !(lvl->n == 2 && (lvl->k <= 3 || (f32 && lvl->k >= 5 && !zero)));
+  }
+
   // one smoothing sweep; `resid` is level-sized scratch for the additive
   // form.  from_zero: u is taken as zero on entry (vmult semantics); the
   // forward multiplicative sweep then starts with the colour-0 pass that
@@ -322,10 +337,7 @@ namespace
         return;
       }
     const long e = timer ? timer->tic_launch() : -1;
-    // (a lone patch of high degree in FP32 is solved sooner on the matrix
-    // cores: Q7 8.4 against 12.5 us, Q6 7.9 against 9.9)
-    const bool lone = lvl->n == 2 && lvl->prec == GTPS_FP32 && lvl->k >= 6 && !from_zero;
-    if (lvl->dim == 3 && row_sweeps_on() && !lone)
+    if (lvl->dim == 3 && row_sweeps_on() && rows_pay(lvl, from_zero && variant == GTPS_MULT_FWD))
       {
         // two colours per launch
         const bool rev = variant == GTPS_MULT_REV;

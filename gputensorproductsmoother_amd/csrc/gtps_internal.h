@@ -209,8 +209,9 @@ namespace gtps
   struct Tuning
   {
     // The knobs up to mfma_waves choose among the kernels of one colour:
-    // 3D additive smoothing, a lone patch of degree 6 or 7 in FP32, and
-    // 3D multiplicative sweeps once one of them is changed (row_sweeps).
+    // 3D additive smoothing, a lone patch (degree 1 to 3; 5 to 7 in FP32
+    // unless the sweep starts from zero), and 3D multiplicative sweeps once
+    // one of them is changed (row_sweeps).
     // Smoother colours with at most this many patches use the single-patch
     // kernel, larger ones the multi-patch kernel (k <= 3).  Measured on
     // MI355X at 64^3 Q3 the single-patch kernel is at least as fast on every

@@ -118,7 +118,10 @@ const char *gtps_version(void);
  *                           16^3); 0: the LDS/FMA kernel.
  *   "row_sweeps"            1 (default): 3D multiplicative sweeps smooth the
  *                           two colours of equal y and z parity in one
- *                           launch, one work-group per x-row of patches;
+ *                           launch, one work-group per x-row of patches,
+ *                           where that is faster (not on two cells per
+ *                           direction with degree 1 to 3, or 5 to 7 in FP32
+ *                           unless the sweep starts from zero);
  *                           0, or any other value than the default of
  *                           small_colour_patches, group_min_patches,
  *                           patches_per_wave, group_waves, row_staged,

@@ -275,6 +275,45 @@ def test_smoother_row_kernel(core, ctx, k, level, variant, prec):
     assert rel_err(out[1], ref) < tol
 
 
+# (k, level, precision, sweep): two colours per launch or one
+ROW_ROUTES = [(1, 1, "fp32", "fwd", 0), (3, 1, "fp64", "rev", 0), (2, 1, "fp64", "zero", 0),
+              (3, 1, "fp32", "revzero", 0), (4, 1, "fp32", "fwd", 1), (4, 1, "fp64", "zero", 1),
+              (5, 1, "fp32", "rev", 0), (6, 1, "fp32", "revzero", 0), (7, 1, "fp32", "fwd", 0),
+              (7, 1, "fp32", "zero", 1), (7, 1, "fp64", "fwd", 1), (1, 2, "fp32", "fwd", 1)]
+
+
+@pytest.mark.parametrize("k,level,prec,sweep,rows", ROW_ROUTES)
+def test_smoother_row_rule(core, ctx, k, level, prec, sweep, rows):
+    """Where one launch per colour is the faster one it runs: the default
+    sweep has the bits of row_sweeps = 0 there and other bits elsewhere, and
+    agrees with the oracle."""
+    _announce("smoother-rule", k, level, prec, sweep)
+    g = rng(level * 19 + k)
+    N = n_dofs(3, k, level)
+    b, u = g.uniform(-1, 1, (2, N))
+    if prec == "fp32":
+        u = u.astype(np.float32).astype(np.float64)
+        b = b.astype(np.float32).astype(np.float64)
+    rev, zero = sweep.startswith("rev"), sweep.endswith("zero")
+    op = core.LaplaceOperator(ctx, 3, k, level, _dt(prec))
+    sm = core.PatchSmoother(op, core.PatchSmoother.MULTIPLICATIVE_REVERSE if rev
+                            else core.PatchSmoother.MULTIPLICATIVE)
+    out = []
+    for on in (1, 0):
+        prev = core.set_tuning("row_sweeps", on)
+        try:
+            ud = _to_dev(u, prec)
+            (sm.vmult if zero else sm.step)(ud, _to_dev(b, prec))
+            torch.cuda.synchronize()
+        finally:
+            core.set_tuning("row_sweeps", prev)
+        out.append(ud.cpu().numpy())
+    assert np.array_equal(out[0], out[1]) == (not rows)
+    ref = O.smoother_step(3, k, level, b, np.zeros(N) if zero else u,
+                          variant=O.MULT_REV if rev else O.MULT_FWD, relax=1.0)
+    assert rel_err(out[0], ref) < TOL[prec] * (20 if prec == "fp32" else 1)
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("path", ["box", "march"])
 @pytest.mark.parametrize("k,level", [(1, 3), (2, 3), (3, 2), (3, 4), (4, 3), (3, 5), (5, 2), (6, 2), (7, 2)])
