@@ -274,12 +274,17 @@ namespace
   // onto u Q1 3.0 / 2.2, Q3 4.4 / 3.2 (FP64 5.3 / 3.7), Q4 5.5 / 6.3 (FP64
   // 6.7 / 8.6), Q7 FP64 19.3 / 24.0, and against the matrix cores in FP32 Q5
   // 7.4 / 7.2, Q6 9.8 / 7.3, Q7 12.3 / 7.8; from zero Q1 2.5 / 2.1, Q3 3.4 /
-  // 3.0 (FP64 3.8 / 3.2), Q4 4.1 / 8.1, Q5 5.8 / 9.0, Q7 8.1 / 9.7.
+  // 3.0 (FP64 3.8 / 3.2), Q4 4.1 / 8.1, Q5 5.8 / 9.0, Q7 8.1 / 9.7.  Q7 FP32
+  // on 16 cells: 112 / 104 onto u (49 to 64 rows on 256 CUs, where a colour's
+  // 343 to 512 patches fill them), 108 / 110 from zero; Q7 FP32 on 8 cells
+  // 60 / 65, on 32 261 / 541, Q6 FP32 on 16 91 / 94, Q7 FP64 249 / 387.
   bool
   rows_pay(const gtps_level *lvl, bool zero)
   {
     const bool f32 = lvl->prec == GTPS_FP32;
-    return !(lvl->n == 2 && (lvl->k <= 3 || (f32 && lvl->k >= 5 && !zero)));
+    if (lvl->n == 2)
+      return !(lvl->k <= 3 || (f32 && lvl->k >= 5 && !zero));
+    return !(f32 && lvl->k == 7 && lvl->n == 16 && !zero);
   }
 
   // one smoothing sweep; `resid` is level-sized scratch for the additive

@@ -210,8 +210,9 @@ namespace gtps
   {
     // The knobs up to mfma_waves choose among the kernels of one colour:
     // 3D additive smoothing, a lone patch (degree 1 to 3; 5 to 7 in FP32
-    // unless the sweep starts from zero), and 3D multiplicative sweeps once
-    // one of them is changed (row_sweeps).
+    // unless the sweep starts from zero), degree 7 in FP32 on 16 cells onto
+    // u, and 3D multiplicative sweeps once one of them is changed
+    // (row_sweeps).
     // Smoother colours with at most this many patches use the single-patch
     // kernel, larger ones the multi-patch kernel (k <= 3).  Measured on
     // MI355X at 64^3 Q3 the single-patch kernel is at least as fast on every

@@ -120,8 +120,9 @@ const char *gtps_version(void);
  *                           two colours of equal y and z parity in one
  *                           launch, one work-group per x-row of patches,
  *                           where that is faster (not on two cells per
- *                           direction with degree 1 to 3, or 5 to 7 in FP32
- *                           unless the sweep starts from zero);
+ *                           direction with degree 1 to 3, nor, unless the
+ *                           sweep starts from zero, in FP32 with degree 5
+ *                           to 7 there and degree 7 on 16 cells);
  *                           0, or any other value than the default of
  *                           small_colour_patches, group_min_patches,
  *                           patches_per_wave, group_waves, row_staged,
