@@ -257,17 +257,23 @@ namespace gtps
   } // namespace
 
   // The tiles recompute the patches and nodes they share, which costs more than
-  // the launches saved once a level fills the GPU.  Measured on MI355X, us per
-  // sweep, this / per colour (from zero): Q2 128^2 FP32 8.6 / 17 (6 / 19),
-  // 512^2 29 / 22 (17 / 27), Q5 128^2 18 / 28 (10 / 31), 512^2 172 / 112
-  // (106 / 124), 1024^2 699 / 383 (414 / 403); FP64 Q2 512^2 33 / 28 (19 /
-  // 35), Q3 512^2 51 / 67 (28 / 80), Q7 512^2 487 / 774 (307 / 797).
+  // the launches saved once a level fills the GPU; FP64 gains all the same
+  // where the per-colour kernel is slow (degree 3 and from 5 on, not 4, whose
+  // tile of 2 x 2 cells recomputes 9 patches for 4).  Measured on MI355X in a
+  // graph, us per sweep, this / per colour (from zero): Q2 128^2 FP32 6.5 / 17
+  // (4.5 / 20), 512^2 29 / 22 (18 / 27), Q5 128^2 18.9 / 27.9 (10.9 / 31),
+  // 512^2 172 / 112 (106 / 125), 1024^2 699 / 383 (414 / 403), Q4 512^2 from
+  // zero 79.2 / 76.9; FP64 Q2 512^2 33 / 28 (20 / 36), Q3 512^2 55 / 69 (31 /
+  // 80), 2048^2 812 / 977, Q4 256^2 49 / 48 (27 / 56), 512^2 157 / 134 (85 /
+  // 145), 1024^2 645 / 502 (329 / 526), 4096^2 10253 / 8395 (6368 / 8801), Q5
+  // 1024^2 966 / 1014, 2048^2 3858 / 3909, Q7 512^2 485 / 775 (306 / 797).
   bool
   additive2d_pays(const gtps_level *lvl, bool zero)
   {
+    const bool f64 = lvl->prec == GTPS_FP64;
     if (zero)
-      return lvl->N <= 10000000 || lvl->prec == GTPS_FP64;
-    return lvl->N <= 600000 || (lvl->prec == GTPS_FP64 && lvl->k >= 3);
+      return f64 || lvl->N <= (lvl->k == 4 ? 2000000 : 10000000);
+    return lvl->N <= 600000 || (f64 && lvl->k >= 3 && lvl->k != 4);
   }
 
   void

@@ -569,6 +569,35 @@ def test_additive_2d_one_launch(core, ctx, k, level, zero, prec):
         assert rel_err(ud.cpu().numpy(), ref) < tol
 
 
+@pytest.mark.parametrize("k,level,prec,zero,one", [
+    (4, 8, "fp64", False, 0), (4, 8, "fp64", True, 1), (4, 7, "fp64", False, 1),
+    (3, 8, "fp64", False, 1), (3, 9, "fp64", False, 1), (5, 8, "fp64", False, 1),
+    (4, 9, "fp32", True, 0), (3, 9, "fp32", True, 1), (3, 9, "fp32", False, 0)])
+def test_additive_2d_rule(core, ctx, k, level, prec, zero, one):
+    """2D additive sweeps take one launch where it is the faster form: the
+    default has the bits of row_sweeps = 0 exactly where it does not."""
+    _announce("additive-2d-rule", k, level, prec, zero)
+    g = torch.Generator(device="cuda:0").manual_seed(level * 13 + k)
+    op = core.LaplaceOperator(ctx, 2, k, level, _dt(prec))
+    sm = core.PatchSmoother(op, core.PatchSmoother.ADDITIVE, 0.4)
+    b, u = (torch.rand(op.n_dofs, generator=g, device="cuda:0", dtype=_dt(prec))
+            for _ in range(2))
+    out = []
+    for on in (1, 0):
+        v = u.clone()
+        torch.cuda.synchronize()
+        prev = core.set_tuning("row_sweeps", on)
+        try:
+            (sm.vmult if zero else sm.step)(v, b)
+        finally:
+            core.set_tuning("row_sweeps", prev)
+        torch.cuda.synchronize()
+        out.append(v)
+    assert torch.equal(*out) == (not one)
+    tol = TOL[prec] * (20 if prec == "fp32" else 1)
+    assert (out[0] - out[1]).abs().max() <= tol * out[1].abs().max()
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("dim,k,level", [(3, 5, 5), (3, 6, 3), (3, 7, 4), (2, 1, 8), (2, 3, 6),
                                          (2, 7, 5)])
