@@ -598,12 +598,28 @@ namespace gtps
             GTPS_LAUNCH_CHECK();
             return;
           }
-      // rows per work-group of the restriction's last pass: several once
-      // there are work-groups enough (2D Q2 1024^2 restriction: 37 us with 128
-      // of 8 rows, 15 us with one row each)
+      // Restriction: rows per work-group of the last pass, several once there
+      // are work-groups enough (2D Q2 1024^2: 37 us with 128 of 8 rows, 15 us
+      // with one row each) and as long as four work-groups share a CU's LDS
       const long long rows = dim == 3 ? (long long)Nc1 * Nc1 : Nc1;
-      const int       rr   = (int)std::max<long long>(1, std::min<long long>(8, rows / 2048));
-      const size_t    lds  = (size_t)rr * Nf1 * sizeof(T);
+      const size_t    line_bytes = Nf1 * sizeof(T);
+      const int       rr  = (int)std::max<long long>(
+        1, std::min<long long>(std::min<long long>(8, rows / 2048), 40960 / (long long)line_bytes));
+      const size_t    lds = rr * line_bytes;
+      // One thread per coarse node instead where the line passes are the
+      // slower form: meshes of few cells (a line's 4k loads are one chain),
+      // and low degrees on rows of which a CU holds few.  Measured on MI355X
+      // in a graph, us, line passes / per node: 2D Q3 4^2 fine cells 5.1 /
+      // 4.5, Q7 16^2 7.0 / 6.9 (FP64 8.5 / 7.9), 32^2 FP64 8.8 / 8.4, 64^2 8.9
+      // / 9.9, Q1 16^2 4.3 / 3.7, 32^2 4.2 / 4.3; 3D Q7 4^3 and 8^3 11.8 / 10.1
+      // and 12.6 / 10.7, 16^3 18 / 24, Q6 8^3 8.7 / 10; 2D Q1 FP64 2048^2 (16
+      // KB a row) 22 / 22, 4096^2 68 / 60, 8192^2 398 / 260, FP32 8192^2 218 /
+      // 198, Q2 FP64 4096^2 (66 KB) 394 / 423, 8192^2 2377 / 1686, Q3 FP64
+      // 4096^2 (98 KB) 1198 / 1275, Q4 4096^2 (131 KB) 2053 / 2852.
+      constexpr int  few3 = K == 7 ? 4 : 0, few2 = K == 7 ? 16 : K == 1 ? 8 : 2;
+      constexpr int  most = (K == 1 ? 24 : K == 2 ? 80 : 160) * 1024;
+      const bool     lines = nc > (dim == 3 ? few3 : few2) && lds <= most && nc < 65535 &&
+                         Nc1 < 65535;
       if (prolong)
         {
           int e0[3] = {Nc1, Nc1, dim == 3 ? Nc1 : 1};
@@ -619,7 +635,7 @@ namespace gtps
               pass<K, T, true, false, 1>(s, t2, fine, tab, dim, 2, e2, e3, nc, Nc1);
             }
         }
-      else if (nc < 65535 && Nc1 < 65535 && lds <= 160 * 1024)
+      else if (lines)
         {
           auto line = [&](const T *in, T *out, long long inner, int outer) {
             hipLaunchKernelGGL((restrict_line_kernel<K, T>),
@@ -654,7 +670,7 @@ namespace gtps
         }
       else
         {
-          // rows beyond the LDS or the grid: one thread per coarse node
+          // one thread per coarse node
           int e0[3] = {Nf1, Nf1, dim == 3 ? Nf1 : 1};
           int e1[3] = {Nc1, Nf1, dim == 3 ? Nf1 : 1};
           int e2[3] = {Nc1, Nc1, dim == 3 ? Nf1 : 1};
