@@ -1197,7 +1197,7 @@ namespace gtps
               return;
             }
           if (relax == 1.0 && tuning().row_sweeps != 0 &&
-              dg_rows_fit(K, lvl->prec, n))
+              dg_rows_fit(K, lvl->prec, n, nvec))
             {
               for (int sw = 0; sw < n_sweeps; ++sw)
                 launch_dg_rows(lvl, u, b, ((first == GTPS_MULT_REV ? 1 : 0) + sw) & 1, nvec);

@@ -490,20 +490,38 @@ namespace gtps
     }
   } // namespace
 
-  // Measured on MI355X, us per sweep, three colours per launch / one: FP32 k =
-  // 2 24^3 99 / 144, k = 4 6^3 139 / 175, 12^3 182 / 178, 24^3 257 / 263 for
-  // one vector (64 rows a launch on 256 CUs) and ~310 / 700 for four, k = 6
-  // 9^3 331 / 367, 12^3 415 / 367; FP64 k = 2 12^3 109 / 139, k = 4 8^3 215 /
-  // 215, 12^3 249 / 213.  The rule does not look at the number of vectors: a
-  // batch and a single solve round alike.
+  // Where three colours per launch are the faster form for nvec vectors at
+  // once.  A row is one work-group whose time grows with n, while a colour
+  // takes the time of one patch as long as its work-groups fit the 256 CUs at
+  // once; with the cheaper local solve of low degrees the launches saved
+  // decide on every mesh.  Measured on MI355X in a graph, us per sweep, rows /
+  // colours, one vector (four): FP32 k = 2 24^3 91 / 136 (97 / 211), k = 3
+  // 12^3 111 / 136, 20^3 135 / 152, k = 4 6^3 140 / 170 (141 / 173), 10^3 169
+  // / 171, 12^3 180 / 171 (184 / 182), 14^3 189 / 178 (197 / 235), 16^3 209 /
+  // 179 (215 / 256), 19^3 230 / 184 (241 / 431), 24^3 267 / 251 (289 / 717),
+  // 28^3 297 / 350, k = 5 11^3 247 / 253, 14^3 293 / 254 (306 / 428), 19^3
+  // 348 / 265 (368 / 956), 24^3 420 / 503, k = 6 9^3 323 / 358, 12^3 415 /
+  // 367; FP64 k = 2 12^3 107 / 132, k = 3 12^3 154 / 160, 16^3 179 / 162 (184
+  // / 233), 19^3 188 / 165 (197 / 376), 24^3 210 / 229 (231 / 628), k = 4 8^3
+  // 211 / 209, 12^3 249 / 213, k = 5 7^3 361 / 365, 8^3 393 / 366.
   bool
-  dg_rows_fit(int k, int prec, int n)
+  dg_rows_fit(int k, int prec, int n, int nvec)
   {
     const bool   f32  = prec == GTPS_FP32;
     const size_t size = row_dispatch(k, [&](auto kk) {
       return (size_t)DR<decltype(kk)::value>::size(n) * (f32 ? 4 : 8);
     });
-    return n >= 5 && size <= 160 * 1024 && (f32 ? k <= 5 || n <= 9 : k <= 3 || n <= 8);
+    const int largest = f32 ? (k <= 5 ? n : 9) : (k <= 3 ? n : k == 4 ? 8 : 7);
+    if (n < 5 || size > 160 * 1024 || n > largest)
+      return false;
+    // degrees and meshes on which the colours win while they fit the chip
+    const int from = f32 ? (k == 4 ? 11 : k == 5 ? 12 : n + 1) : (k == 3 ? 15 : n + 1);
+    if (n < from)
+      return true;
+    const long long side = (n + 1) / 3;  // of the largest colour
+    const bool one_round = side * side * side * nvec <= 256 ||
+                           (nvec == 1 && n <= (f32 && k == 4 ? 24 : 20));
+    return !one_round;
   }
 
   void

@@ -334,8 +334,9 @@ namespace gtps
   void dg_level_reserve(gtps_dg_level *lvl, int nb);
   bool dg_supported(int k, int prec);
   // dg_row.hip: one undamped sweep (reverse: colours descending), three
-  // x-colours per launch; the mesh must fit (one row's data in LDS)
-  bool dg_rows_fit(int k, int prec, int n);
+  // x-colours per launch; dg_rows_fit: it is faster than one colour per
+  // launch for nvec vectors at once, and one row's data fits the LDS
+  bool dg_rows_fit(int k, int prec, int n, int nvec);
   void launch_dg_rows(const gtps_dg_level *lvl, void *u, const void *b, bool reverse, int nvec);
   // Every DG launcher takes a batch of nb contiguous vectors (stride lvl->N
   // on the level, the coarse level's N for coarse operands); one launch.

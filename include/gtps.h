@@ -129,10 +129,14 @@ const char *gtps_version(void);
  *                           mfma_smoother or mfma_waves: one launch per
  *                           colour with the kernels these knobs choose.
  *                           DG sweeps without damping: 1 three x-colours
- *                           per launch where a row fits the LDS, 0 one;
+ *                           per launch where that is faster, which depends
+ *                           on the number of vectors smoothed together, 0
+ *                           one (a batch then has the bits of its single
+ *                           solves on every mesh; with 1 it has them where
+ *                           both take the same launches);
  *                           2D additive sweeps: 1 residual and all patches
- *                           in one launch, 0 one for the residual and one
- *                           per colour;
+ *                           in one launch where that is faster, 0 one for
+ *                           the residual and one per colour;
  *   "mfma_waves"            matrix-core smoother wavefronts per patch: 4,
  *                           8 (default) or 16.
  * Results do not depend on the knobs beyond round-off.  No reference

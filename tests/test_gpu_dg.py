@@ -149,6 +149,67 @@ def test_dg_smoother_rows(core, ctx, k, n, reverse, prec):
         assert rel_err(got, ref) < TOL_SMOOTH[prec]
 
 
+# (k, n, precision): three x-colours per launch or one, for a single vector
+ROW_ROUTES = [(3, 12, "fp32", 1), (4, 10, "fp32", 1), (4, 11, "fp32", 0), (4, 16, "fp32", 0),
+              (4, 24, "fp32", 0), (4, 25, "fp32", 1), (5, 11, "fp32", 1), (5, 12, "fp32", 0),
+              (5, 20, "fp32", 0), (5, 21, "fp32", 1), (6, 9, "fp32", 1), (6, 10, "fp32", 0),
+              (3, 14, "fp64", 1), (3, 16, "fp64", 0), (3, 21, "fp64", 1), (4, 8, "fp64", 1),
+              (5, 7, "fp64", 1), (5, 8, "fp64", 0)]
+
+
+@pytest.mark.parametrize("k,n,prec,rows", ROW_ROUTES)
+def test_dg_smoother_row_rule(core, ctx, k, n, prec, rows):
+    """A sweep of one vector takes the form that is faster for it: the
+    default has the bits of row_sweeps = 0 where that is one colour per
+    launch, and the two forms agree."""
+    _announce("dg-row-rule", k, n, prec)
+    op = core.DGOperator(ctx, 3, k, n, _prec(core, prec))
+    g = torch.Generator(device="cuda:0").manual_seed(10 * n + k)
+    b, u = (torch.rand(op.n_dofs, generator=g, device="cuda:0", dtype=_dt(prec)) - 0.5
+            for _ in range(2))
+    out = []
+    for on in (1, 0):
+        v = u.clone()
+        torch.cuda.synchronize()
+        prev = core.set_tuning("row_sweeps", on)
+        try:
+            op.smoother_step(v, b)
+        finally:
+            core.set_tuning("row_sweeps", prev)
+        torch.cuda.synchronize()
+        out.append(v)
+    assert torch.equal(*out) == (not rows)
+    assert rel_err(_host(out[0]), _host(out[1])) < TOL_SMOOTH[prec]
+
+
+def test_dg_batch_takes_rows_where_one_vector_does_not(core, ctx):
+    """Q4 on 11^3 cells: five vectors are smoothed in rows, a single one colour
+    by colour. Both solve to the tolerance, equal rows of the batch are
+    bitwise equal, and with row_sweeps = 0 they are the single solve's
+    bits."""
+    k, n = 4, 11
+    _announce("dg-batch-rows", k, n)
+    mg = core.DGMultigrid(ctx, 3, k, n, 0, core.FP32)
+    b = _dev(rng(64).uniform(-1, 1, mg.n_dofs))
+    B = torch.stack([b] * 5)
+    sols = {}
+    for on in (1, 0):
+        prev = core.set_tuning("row_sweeps", on)
+        try:
+            x, it, rel, _ = mg.solve_cg(b, rtol=1e-8)
+            X, its, rels = mg.solve_cg_batch(B, rtol=1e-8)
+        finally:
+            core.set_tuning("row_sweeps", prev)
+        torch.cuda.synchronize()
+        assert rel <= 1e-8 and max(rels) <= 1e-8 and its == [it] * 5
+        assert all(torch.equal(X[0], X[j]) for j in range(1, 5))
+        sols[on] = x.clone(), X[0].clone()
+    assert torch.equal(*sols[0])
+    assert torch.equal(sols[1][0], sols[0][0]) and not torch.equal(*sols[1])
+    # two solutions with residuals of 1e-8 of the start's
+    assert rel_err(_host(sols[1][1]), _host(sols[1][0])) < 1e-6
+
+
 def test_dg_smoother_reduces_error(core, ctx):
     """One symmetric sweep pair contracts the A-norm error of A u = b."""
     _announce("dg-smoother-contract", 3, 6)
