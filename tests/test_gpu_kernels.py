@@ -276,6 +276,30 @@ def test_smoother_row_kernel(core, ctx, k, level, variant, prec):
     assert rel_err(out[1], ref) < tol
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("variant", ["fwd", "rev", "zero"])
+@pytest.mark.parametrize("k,level", [(1, 3), (3, 2), (3, 6), (5, 3), (7, 3)])
+def test_smoother_rows_rim_of_rhs(core, ctx, k, level, variant, prec):
+    """The right-hand side on the Dirichlet nodes, which the row kernel reads
+    along with its columns, reaches no result: NaN there changes no bit."""
+    _announce("smoother-rim", k, level, variant, prec)
+    g = torch.Generator(device="cuda:0").manual_seed(level * 23 + k)
+    op = core.LaplaceOperator(ctx, 3, k, level, _dt(prec))
+    sm = core.PatchSmoother(op, core.PatchSmoother.MULTIPLICATIVE_REVERSE if variant == "rev"
+                            else core.PatchSmoother.MULTIPLICATIVE)
+    b, u = (torch.rand(op.n_dofs, generator=g, device="cuda:0", dtype=_dt(prec))
+            for _ in range(2))
+    out = []
+    for rim in (0.0, float("nan")):
+        op.set_constrained_values(b, rim)
+        v = u.clone()
+        torch.cuda.synchronize()
+        (sm.vmult if variant == "zero" else sm.step)(v, b)
+        torch.cuda.synchronize()
+        out.append(v)
+    assert torch.isfinite(out[0]).all() and torch.equal(*out)
+
+
 # (k, level, precision, sweep): two colours per launch or one
 ROW_ROUTES = [(1, 1, "fp32", "fwd", 0), (3, 1, "fp64", "rev", 0), (2, 1, "fp64", "zero", 0),
               (3, 1, "fp32", "revzero", 0), (4, 1, "fp32", "fwd", 1), (4, 1, "fp64", "zero", 1),
