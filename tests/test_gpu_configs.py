@@ -140,9 +140,10 @@ def test_c2_workload(core, ctx):
 
 def test_c3_workload(core, ctx):
     """C3: 3D Q7 on 32^3 cells (N = 225^3), f = 1, CG to 1e-8: the FP32
-    V-cycle with the matrix-core smoother and with the LDS/FMA smoother,
-    and FP64 everywhere, 5 iterations each, within 1e-8 of a GPU FP64 solve
-    to 1e-12; true residuals and the full-size operator from the oracle."""
+    V-cycle with the row smoother (the default), with the matrix-core one and
+    with the LDS/FMA one (one launch per colour), and FP64 everywhere, 5
+    iterations each, within 1e-8 of a GPU FP64 solve to 1e-12; true residuals
+    and the full-size operator from the oracle."""
     dim, k, level = 3, 7, 5
     _announce("C3", dim, k, level)
     b = O.rhs_assembled(dim, k, level, O.RHS_CONST)
@@ -154,20 +155,26 @@ def test_c3_workload(core, ctx):
     assert rel_ref <= 1e-12
     assert _true_relres(b, O.laplace_vmult(dim, k, level, x_ref)) <= 1e-11
     sols = {}
-    for mf in (1, 0):
-        prev = core.set_tuning("mfma_smoother", mf)
+    for name, rows, mf in (("rows", 1, 1), ("matrix cores", 0, 1), ("LDS/FMA", 0, 0)):
+        prev = core.set_tuning("row_sweeps", rows), core.set_tuning("mfma_smoother", mf)
         try:
-            _announce("C3 FP32 smoother", "matrix cores" if mf else "LDS/FMA")
-            sols[mf] = _solve_forms(core, ctx, dim, k, level, bd, 1e-8, 5, x_ref=x_ref,
-                                    precs=("fp32",))["fp32"]
+            _announce("C3 FP32 smoother", name)
+            sols[name] = _solve_forms(core, ctx, dim, k, level, bd, 1e-8, 5, x_ref=x_ref,
+                                      precs=("fp32",))["fp32"]
         finally:
-            core.set_tuning("mfma_smoother", prev)
+            core.set_tuning("row_sweeps", prev[0])
+            core.set_tuning("mfma_smoother", prev[1])
     _solve_forms(core, ctx, dim, k, level, bd, 1e-8, 5, x_ref=x_ref, precs=("fp64",))
-    for mf, x in sols.items():
+    for name, x in sols.items():
         Ax = O.laplace_vmult(dim, k, level, x.cpu().numpy())
-        assert _true_relres(b, Ax) <= 1.1e-8, mf
-    # the two FP32 smoothers are the same operator up to FP32 round-off
-    assert _rel_l2(sols[1], sols[0]) < PARITY
+        assert _true_relres(b, Ax) <= 1.1e-8, name
+    # the FP32 smoothers are the same operator up to FP32 round-off, in three
+    # orders of summation
+    for name in ("matrix cores", "LDS/FMA"):
+        assert not torch.equal(sols[name], sols["rows"])
+        assert _rel_l2(sols[name], sols["rows"]) < PARITY
+    assert not torch.equal(sols["matrix cores"], sols["LDS/FMA"])
+    assert _rel_l2(sols["matrix cores"], sols["LDS/FMA"]) < PARITY
 
 
 def test_c4_workload(core, ctx, problems):

@@ -376,8 +376,8 @@ def test_vmult_box_and_march_paths(core, ctx, k, level, path, prec):
 def test_smoother_matrix_core_path(core, ctx, k, level, reverse, mfma):
     """3D FP32 multiplicative smoothing of degree 4..7 on the matrix cores
     (v_mfma_f32_16x16x4f32, patches padded to 16^3) with mfma = 4, 8 or 16
-    wavefronts per patch, and on the LDS/FMA kernel (mfma = 0), agree with
-    the oracle (FP32 tolerance x20, relaxation 0.8)."""
+    wavefronts per patch, and on the LDS/FMA kernel (mfma = 0), one launch
+    per colour, agree with the oracle (FP32 tolerance x20, relaxation 0.8)."""
     _announce("smoother-mfma", k, level, reverse, mfma)
     g = rng(level * 11 + k)
     N = n_dofs(3, k, level)
@@ -387,8 +387,8 @@ def test_smoother_matrix_core_path(core, ctx, k, level, reverse, mfma):
     relax = 0.8
     ref = O.smoother_step(3, k, level, b, u, variant=O.MULT_REV if reverse else O.MULT_FWD,
                           relax=relax)
-    prev = core.set_tuning("mfma_smoother", 1 if mfma else 0)
-    prev_waves = core.set_tuning("mfma_waves", mfma or 8)
+    keys = {"row_sweeps": 0, "mfma_smoother": 1 if mfma else 0, "mfma_waves": mfma or 8}
+    prev = {key: core.set_tuning(key, v) for key, v in keys.items()}
     try:
         op = core.LaplaceOperator(ctx, 3, k, level, torch.float32)
         sm = core.PatchSmoother(op, core.PatchSmoother.MULTIPLICATIVE_REVERSE if reverse
@@ -397,8 +397,8 @@ def test_smoother_matrix_core_path(core, ctx, k, level, reverse, mfma):
         sm.step(ud, _to_dev(b, "fp32"))
         torch.cuda.synchronize()
     finally:
-        core.set_tuning("mfma_smoother", prev)
-        core.set_tuning("mfma_waves", prev_waves)
+        for key, v in prev.items():
+            core.set_tuning(key, v)
     assert rel_err(ud.cpu().numpy(), ref) < TOL["fp32"] * 20
 
 
