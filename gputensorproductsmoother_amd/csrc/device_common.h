@@ -177,68 +177,81 @@ namespace gtps
     return (__umulhi(n, f.m) + n) >> f.s;
   }
 
-      // Fast-diagonalisation transforms in the even/odd eigenbasis (tables
-      // Tab::SE, Tab::SO): t = S^T v with t numbered even vectors first, and
-      // its inverse v = S t.  The reflection symmetry of the eigenvectors
-      // halves the products: K(K) + (K-1)^2 multiply-adds and 2(K-1)
-      // additions instead of (2K-1)^2.
-      template <int K, typename T>
-      __device__ __forceinline__ void
-      fd_fwd(const T *SE, const T *SO, const T (&v)[2 * K - 1], T (&t)[2 * K - 1])
+  // Fast-diagonalisation transforms in the even/odd eigenbasis (tables
+  // Tab::SE, Tab::SO): t = S^T v with t numbered even vectors first, and
+  // its inverse v = S t.  The reflection symmetry of the eigenvectors
+  // halves the products: K(K) + (K-1)^2 multiply-adds and 2(K-1)
+  // additions instead of (2K-1)^2.
+  template <int K, typename T>
+  __device__ __forceinline__ void
+  fd_fwd(const T *SE, const T *SO, const T (&v)[2 * K - 1], T (&t)[2 * K - 1])
+  {
+    constexpr int NI = 2 * K - 1, MH = K - 1, NE = K, NO = K - 1;
+    T e[MH + 1], o[MH > 0 ? MH : 1];
+#pragma unroll
+    for (int i = 0; i < MH; ++i)
       {
-        constexpr int NI = 2 * K - 1, MH = K - 1, NE = K, NO = K - 1;
-        T e[MH + 1], o[MH > 0 ? MH : 1];
-  #pragma unroll
-        for (int i = 0; i < MH; ++i)
-          {
-            e[i] = v[i] + v[NI - 1 - i];
-            o[i] = v[i] - v[NI - 1 - i];
-          }
-        e[MH] = v[MH];
-  #pragma unroll
-        for (int q = 0; q < NE; ++q)
-          {
-            T s = 0;
-  #pragma unroll
-            for (int i = 0; i <= MH; ++i)
-              s += SE[i * NE + q] * e[i];
-            t[q] = s;
-          }
-  #pragma unroll
-        for (int q = 0; q < NO; ++q)
-          {
-            T s = 0;
-  #pragma unroll
-            for (int i = 0; i < MH; ++i)
-              s += SO[i * NO + q] * o[i];
-            t[NE + q] = s;
-          }
+        e[i] = v[i] + v[NI - 1 - i];
+        o[i] = v[i] - v[NI - 1 - i];
       }
+    e[MH] = v[MH];
+#pragma unroll
+    for (int q = 0; q < NE; ++q)
+      {
+        T s = 0;
+#pragma unroll
+        for (int i = 0; i <= MH; ++i)
+          s += SE[i * NE + q] * e[i];
+        t[q] = s;
+      }
+#pragma unroll
+    for (int q = 0; q < NO; ++q)
+      {
+        T s = 0;
+#pragma unroll
+        for (int i = 0; i < MH; ++i)
+          s += SO[i * NO + q] * o[i];
+        t[NE + q] = s;
+      }
+  }
 
-      template <int K, typename T>
-      __device__ __forceinline__ void
-      fd_inv(const T *SE, const T *SO, const T (&t)[2 * K - 1], T (&v)[2 * K - 1])
+  template <int K, typename T>
+  __device__ __forceinline__ void
+  fd_inv(const T *SE, const T *SO, const T (&t)[2 * K - 1], T (&v)[2 * K - 1])
+  {
+    constexpr int NI = 2 * K - 1, MH = K - 1, NE = K, NO = K - 1;
+#pragma unroll
+    for (int i = 0; i < MH; ++i)
       {
-        constexpr int NI = 2 * K - 1, MH = K - 1, NE = K, NO = K - 1;
-  #pragma unroll
-        for (int i = 0; i < MH; ++i)
-          {
-            T pe = 0, po = 0;
-  #pragma unroll
-            for (int q = 0; q < NE; ++q)
-              pe += SE[i * NE + q] * t[q];
-  #pragma unroll
-            for (int q = 0; q < NO; ++q)
-              po += SO[i * NO + q] * t[NE + q];
-            v[i]          = pe + po;
-            v[NI - 1 - i] = pe - po;
-          }
-        T pm = 0;
-  #pragma unroll
+        T pe = 0, po = 0;
+#pragma unroll
         for (int q = 0; q < NE; ++q)
-          pm += SE[MH * NE + q] * t[q];
-        v[MH] = pm;
+          pe += SE[i * NE + q] * t[q];
+#pragma unroll
+        for (int q = 0; q < NO; ++q)
+          po += SO[i * NO + q] * t[NE + q];
+        v[i]          = pe + po;
+        v[NI - 1 - i] = pe - po;
       }
+    T pm = 0;
+#pragma unroll
+    for (int q = 0; q < NE; ++q)
+      pm += SE[MH * NE + q] * t[q];
+    v[MH] = pm;
+  }
+
+  // table address hidden from the optimiser: the entries are loaded (scalar)
+  // for this use instead of being kept live and spilled
+  template <typename T>
+  using ConstP = const T __attribute__((address_space(4))) *;
+  template <typename T>
+  __device__ __forceinline__ ConstP<T>
+  here(const T *p)
+  {
+    ConstP<T> c = (ConstP<T>)p;
+    asm volatile("" : "+s"(c));
+    return c;
+  }
 
   __device__ __forceinline__ int
   linear_block_id()

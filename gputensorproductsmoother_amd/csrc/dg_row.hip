@@ -41,19 +41,6 @@ namespace gtps
       __host__ __device__ static int size(int n) { return CT(n) + 10 * NI; }
     };
 
-    // table address hidden from the optimiser: entries are loaded (scalar)
-    // for this use instead of being kept live and spilled
-    template <typename T>
-    using ConstP = const T __attribute__((address_space(4))) *;
-    template <typename T>
-    __device__ __forceinline__ ConstP<T>
-    here(const T *p)
-    {
-      ConstP<T> c = (ConstP<T>)p;
-      asm volatile("" : "+s"(c));
-      return c;
-    }
-
     // t_q = sum_a A[a][q] v_a, and v_a = sum_q A[a][q] t_q
     template <int NI, typename T>
     __device__ __forceinline__ void

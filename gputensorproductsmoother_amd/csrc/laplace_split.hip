@@ -29,18 +29,6 @@ namespace gtps
       static size_t lds(int n) { return (size_t)2 * ROWS * ((K * n + 1) | 1) * sizeof(T); }
     };
 
-    // table rows loaded (scalar) where they are used
-    template <typename T>
-    using ConstP = const T __attribute__((address_space(4))) *;
-    template <typename T>
-    __device__ __forceinline__ ConstP<T>
-    here(const T *p)
-    {
-      ConstP<T> c = (ConstP<T>)p;
-      asm volatile("" : "+s"(c));
-      return c;
-    }
-
     // a = M_y M_x u, c = (K_y M_x + M_y K_x) u on the rows 0 < y < N1 - 1 of
     // plane blockIdx.y; work-group = CY cells along y, whole rows in LDS.
     // n lanes of one wavefront share a row (n <= 64), so the row's products

@@ -69,16 +69,6 @@ namespace gtps
     // thread instead of 4.0k, k = 5 FP64 2.3k instead of 1.9k.  Below that
     // the repeated loads cost more (k = 3 FP32 122 instead of 106 us a
     // sweep at 64^3).
-    template <typename T>
-    using ConstP = const T __attribute__((address_space(4))) *;
-    template <typename T>
-    __device__ __forceinline__ ConstP<T>
-    here(const T *p)
-    {
-      ConstP<T> c = (ConstP<T>)p;
-      asm volatile("" : "+s"(c));
-      return c;
-    }
     template <int K, typename T>
     constexpr bool LAUNDER = sizeof(T) == 8 ? K >= 5 : K >= 6;
     template <int K, typename T>
