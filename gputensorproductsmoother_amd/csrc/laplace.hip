@@ -921,13 +921,12 @@ namespace gtps
   {
     if (lvl->coef)
       return launch_coeff_apply(lvl, y, x, b, fused_dot, false);
-    // two launches where they are faster, unless a knob of the one-launch
-    // kernels was changed or the launch would bind the level's scratch into a
-    // caller's graph
+    // two launches where they are faster (degree 5 on), unless the box kernel
+    // was asked for on this level, a knob of the z-marching kernel was changed
+    // or the launch would bind the level's scratch into a caller's graph
     const Tuning t, &cur = tuning();
-    if (lvl->split && cur.box_vmult_max_n == t.box_vmult_max_n &&
-        cur.vmult_zdiv == t.vmult_zdiv && cur.vmult_tile == t.vmult_tile &&
-        !callers_capture(lvl->ctx))
+    if (lvl->split && lvl->n > cur.box_vmult_max_n / 2 && cur.vmult_zdiv == t.vmult_zdiv &&
+        cur.vmult_tile == t.vmult_tile && !callers_capture(lvl->ctx))
       return launch_laplace_split(lvl, y, x, b, fused_dot);
     if (lvl->prec == GTPS_FP32)
       return launch_t<float>(lvl, y, x, b, fused_dot);

@@ -104,12 +104,20 @@ const char *gtps_version(void);
  *                           level-2 smoothing and level-1 solve.
  *   "vmult_zdiv"            z-marching vmult work-group count target: z-chunks
  *                           of ceil(n tx ty / value) cells (default 0: 512
- *                           in FP32, 2048 in FP64, 256 in FP64 at k = 7);
+ *                           in FP32, with chunks of at most 3 cells for
+ *                           degree 1, 2 and 4, 2048 in FP64, 256 in FP64 at
+ *                           k = 7);
  *   "vmult_tile"            z-marching vmult tile for k = 3: 0: 16x8 cells
  *                           and 512 threads, 1: 8x8 and 256, 2: 16x8 and
  *                           256, 3 (default): 0 in FP32, 1 in FP64; for
  *                           k = 7: 0: 8x2 cells and 512 threads, 1: 4x4
- *                           and 1024, 2 and 3 (default): 4x4 and 512;
+ *                           and 1024, 2 and 3 (default): 4x4 and 512.
+ *                           On 32 cells per direction with degree 5 to 7,
+ *                           and on 64 with degree 5 in FP32, the operator
+ *                           takes two launches instead, unless vmult_zdiv
+ *                           or vmult_tile is changed from its default,
+ *                           box_vmult_max_n covers the level, or the call
+ *                           is captured into a caller's graph;
  *   "mfma_smoother"         where a sweep launches colour by colour (see
  *                           row_sweeps), 1 (default): 3D FP32
  *                           multiplicative smoothing of degree 4..7 runs
@@ -351,8 +359,10 @@ int gtps_mg_set_graph(gtps_mg *mg, int enable);
  * include/solver.cuh:1747-1771, filled at 1957-1999) without its per-stage
  * device synchronisations.  `mask` enables groups (bit g = group g):
  *   GTPS_PROF_SMOOTH_FINE   finest-level sweeps, one event pair per sweep,
- *                           counted as its colour launches (so total/count
- *                           is the mean colour-launch time)
+ *                           counted as its launches: 4 of two colours each
+ *                           (row_sweeps), else one per colour; one (from
+ *                           zero) or two for a 2D additive sweep in one
+ *                           launch (total/count is the mean launch time)
  *   GTPS_PROF_SMOOTH_COARSE smoothing sweeps on the coarser levels
  *   GTPS_PROF_RESIDUAL_FINE t = d - A u on the finest level
  *   GTPS_PROF_TRANSFER      restriction and prolongation, all levels

@@ -286,10 +286,10 @@ def test_coefficient_releases_two_launch_scratch(core, ctx):
     op.vmult(z, x)
     torch.cuda.synchronize()
     assert torch.equal(y, z)
-    prev = core.set_tuning("box_vmult_max_n", 15)  # one launch
+    prev = core.set_tuning("vmult_tile", 0)  # one launch
     try:
         op.vmult(y, x)
     finally:
-        core.set_tuning("box_vmult_max_n", prev)
+        core.set_tuning("vmult_tile", prev)
     torch.cuda.synchronize()
     assert not torch.equal(y, z)

@@ -522,6 +522,29 @@ def test_vmult_two_launches(core, ctx, k, level, prec):
     assert rel_err(bd.cpu().numpy(), b - ref) < TOL[prec]
 
 
+@pytest.mark.parametrize("key,value,two", [("box_vmult_max_n", 8, True),
+                                           ("box_vmult_max_n", 63, True),
+                                           ("box_vmult_max_n", 64, False),
+                                           ("vmult_zdiv", 100, False), ("vmult_tile", 0, False)])
+def test_vmult_two_launches_and_knobs(core, ctx, key, value, two):
+    """The two-launch operator gives way to the knobs that ask for another
+    kernel on its level, and to no other: its bits stay or change."""
+    _announce("vmult-two-knobs", key, value)
+    k, level = 5, 5
+    x = _to_dev(rng(72).uniform(-1, 1, n_dofs(3, k, level)), "fp32")
+    op = core.LaplaceOperator(ctx, 3, k, level, torch.float32)
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    op.vmult(y, x)
+    prev = core.set_tuning(key, value)
+    try:
+        op.vmult(z, x)
+    finally:
+        core.set_tuning(key, prev)
+    torch.cuda.synchronize()
+    assert torch.equal(y, z) == two
+    assert (y - z).abs().max() <= TOL["fp32"] * y.abs().max()
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 def test_vmult_captured_by_caller(core, prec):
     """Two graphs that a program records from one operator hold no scratch of
@@ -537,12 +560,12 @@ def test_vmult_captured_by_caller(core, prec):
     y = [torch.empty_like(v) for v in x]
     want = [torch.empty_like(v) for v in x]
     torch.cuda.synchronize()
-    prev = core.set_tuning("box_vmult_max_n", 15)  # any change: one launch
+    prev = core.set_tuning("vmult_tile", 0)  # any change: one launch
     try:
         for v, w in zip(x, want):
             op.vmult(w, v)
     finally:
-        core.set_tuning("box_vmult_max_n", prev)
+        core.set_tuning("vmult_tile", prev)
     torch.cuda.synchronize()
     graphs = []
     for v, w in zip(x, y):
