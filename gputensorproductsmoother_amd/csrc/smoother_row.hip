@@ -201,9 +201,13 @@ namespace gtps
 
       // The right-hand side at the domain's ends and the x face positions that
       // are no face reach no result; read with the rest (inside the box) or
-      // zero.  Either form on every degree is slower: zero Q3 64^3 FP32 95.7
-      // instead of 93.4 us a sweep, read Q7 32^3 FP64 598 instead of 562.
-      constexpr bool ENDS = !LAUNDER<K, T>;
+      // zero, the former set where it is loaded (EARLY) or used.  No form
+      // suits every degree: zero Q3 64^3 FP32 95.7 instead of 93.4 us a sweep,
+      // read Q7 32^3 FP64 598 instead of 562, zero where loaded 575; Q7 32^3
+      // FP32, two sweeps among those of other streams, 415 us zero where
+      // loaded, 427 where used.
+      constexpr bool ENDS  = !LAUNDER<K, T>;
+      constexpr bool EARLY = K == 7 && sizeof(T) == 4;
       constexpr int NB = NI * WX;                       // interior lines by column
       constexpr int TF = 2 * WX + NPOS * NI;            // first face direction
       constexpr int PB = (NB + NT - 1) / NT, PF = (TF + NT - 1) / NT;
@@ -242,6 +246,12 @@ namespace gtps
 #pragma unroll
                   for (int z = 0; z < NI; ++z)
                     rb[pp][z] = p[z * P];
+                }
+              else if (EARLY)
+                {
+#pragma unroll
+                  for (int z = 0; z < NI; ++z)
+                    rb[pp][z] = 0;
                 }
             }
           T fl[ZERO ? 1 : PF][NP], fr[ZERO ? 1 : PF][NP];
@@ -295,7 +305,7 @@ namespace gtps
                   const int x = x0 + col;
                   T        *d = sm + C::FD + y * RS + col;
                   T         tt[NI];
-                  if (ENDS || (x > 0 && x < N1 - 1))
+                  if (ENDS || EARLY || (x > 0 && x < N1 - 1))
                     row_fwd<K>(SE, SO, rb[pp], tt);
                   else
                     {
