@@ -370,7 +370,7 @@ namespace
 
 struct gtps_mg : LaunchTimer
 {
-  gtps_ctx                  *ctx = nullptr;
+  gtps::CtxRef               ctx;
   int                        dim = 3, k = 1, maxl = 1, prec = GTPS_FP32;
   int                        schedule = GTPS_MG_SYMMETRIC;
   double                     relax    = 1.0;
@@ -992,7 +992,7 @@ namespace
 // pairs from zero; FP64 CG on the finest level.
 struct gtps_dg_mg
 {
-  gtps_ctx                     *ctx = nullptr;
+  gtps::CtxRef                  ctx;
   int                           dim = 3, k = 1, n0 = 3, maxl = 0;
   int                           prec = GTPS_FP32, coarse_sweeps = 2;
   double                        pf = 1.0, relax = 1.0;
@@ -1369,6 +1369,34 @@ struct gtps_dg_mg
   }
 };
 
+namespace gtps
+{
+  void
+  ctx_release(gtps_ctx *ctx) noexcept
+  {
+    if (--ctx->refs > 0)
+      return;
+    (void)hipSetDevice(ctx->device);
+    (void)hipStreamSynchronize(ctx->stream);
+    for (auto &kv : ctx->tables)
+      {
+        dfree(kv.second->d64);
+        dfree(kv.second->d32);
+        dfree(kv.second->sep64);
+        dfree(kv.second->sep32);
+      }
+    dfree(ctx->ws.partials);
+    dfree(ctx->ws.scalars);
+    if (ctx->ws.pinned)
+      (void)hipHostFree(ctx->ws.pinned);
+    if (ctx->ws.readback)
+      (void)hipHostFree(ctx->ws.readback);
+    if (ctx->own_stream)
+      (void)hipStreamDestroy(ctx->stream);
+    delete ctx;
+  }
+} // namespace gtps
+
 extern "C"
 {
   const char *
@@ -1425,22 +1453,7 @@ extern "C"
         return;
       (void)hipSetDevice(ctx->device);
       (void)hipStreamSynchronize(ctx->stream);
-      for (auto &kv : ctx->tables)
-        {
-          dfree(kv.second->d64);
-          dfree(kv.second->d32);
-          dfree(kv.second->sep64);
-          dfree(kv.second->sep32);
-        }
-      dfree(ctx->ws.partials);
-      dfree(ctx->ws.scalars);
-      if (ctx->ws.pinned)
-        (void)hipHostFree(ctx->ws.pinned);
-      if (ctx->ws.readback)
-        (void)hipHostFree(ctx->ws.readback);
-      if (ctx->own_stream)
-        (void)hipStreamDestroy(ctx->stream);
-      delete ctx;
+      ctx_release(ctx);
     });
   }
 

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <memory>
 #include <stdexcept>
@@ -102,6 +103,10 @@ namespace gtps
 
 struct gtps_ctx
 {
+  // gtps_ctx_create's reference and one per handle made on the context:
+  // handles may be destroyed after gtps_ctx_destroy (a garbage collector
+  // takes them in any order) and synchronise its stream when they are
+  std::atomic<int>                                        refs{1};
   int                                                     device = 0;
   hipStream_t                                             stream = nullptr;
   bool                                                    own_stream = false;
@@ -112,9 +117,50 @@ struct gtps_ctx
   std::map<int, std::unique_ptr<gtps::DegreeTables>>      tables;
 };
 
+namespace gtps
+{
+  // drops a reference; the last one frees the context (capi.hip)
+  void ctx_release(gtps_ctx *ctx) noexcept;
+
+  // a handle's reference to its context
+  class CtxRef
+  {
+  public:
+    CtxRef()               = default;
+    CtxRef(const CtxRef &) = delete;
+    ~CtxRef() { reset(nullptr); }
+    CtxRef &
+    operator=(const CtxRef &o)
+    {
+      reset(o.p);
+      return *this;
+    }
+    CtxRef &
+    operator=(gtps_ctx *c)
+    {
+      reset(c);
+      return *this;
+    }
+    operator gtps_ctx *() const { return p; }
+    gtps_ctx *operator->() const { return p; }
+
+  private:
+    void
+    reset(gtps_ctx *c)
+    {
+      if (c)
+        ++c->refs;
+      if (p)
+        ctx_release(p);
+      p = c;
+    }
+    gtps_ctx *p = nullptr;
+  };
+} // namespace gtps
+
 struct gtps_level
 {
-  gtps_ctx                *ctx = nullptr;
+  gtps::CtxRef             ctx;
   int                      dim = 3, k = 1, level = 1, n = 2, N1 = 3;
   long long                N   = 0;
   int                      prec = GTPS_FP64;
@@ -172,7 +218,7 @@ struct gtps_smoother
 // X = cx (k+1) + ix, index X + N1 Y + N1^2 Z.
 struct gtps_dg_level
 {
-  gtps_ctx *ctx = nullptr;
+  gtps::CtxRef ctx;
   int       dim = 3, k = 1, n = 2, N1 = 4;
   long long N   = 0;
   int       prec = GTPS_FP64;
@@ -197,7 +243,7 @@ struct gtps_dg_level
 
 struct gtps_transfer
 {
-  gtps_ctx *ctx = nullptr;
+  gtps::CtxRef ctx;
   int       dim = 3, k = 1, min_level = 1, max_level = 1, prec = GTPS_FP64;
   void     *tmp1 = nullptr, *tmp2 = nullptr;
   gtps::DegreeTables *tab = nullptr;

@@ -59,7 +59,8 @@ typedef struct gtps_dg_mg gtps_dg_mg;
 /* ---------------------------------------------------------------- context */
 /* Device selection and stream; replaces the reference's implicit CUDA
  * default stream and findCudaDevice (apps/poisson.cu:488-489).
- * stream == NULL creates a stream owned by the context. */
+ * stream == NULL creates a stream owned by the context.  Handles keep their
+ * context: what gtps_ctx_destroy leaves is freed with the last of them. */
 int gtps_ctx_create(int device, void *stream, gtps_ctx **out);
 int gtps_ctx_destroy(gtps_ctx *ctx);
 int gtps_ctx_synchronize(gtps_ctx *ctx);

@@ -312,3 +312,42 @@ def test_dg_adjoint_loss_on_one_row(core, ctx):
         assert torch.count_nonzero(gB[j]).item() == 0, j
     ref, _, _, _ = O.dg_pcg(3, k, n0, maxl, w, rtol=1e-12)
     assert rel_err(gB[0].cpu().numpy(), ref) < 1e-8
+
+
+def test_handles_outlive_their_context(core):
+    """A closed context serves the handles made on it until the last of them
+    is gone, in any order of destruction: a garbage collector that finds a
+    context and its solvers in one cycle destroys the context first."""
+    import gc
+    _announce("ctx-outlived")
+    k, level = 2, 3
+    cx = core.Context(0)
+    mg = core.MultigridSolvers(cx, 3, k, level, torch.float32)
+    dg = core.DGMultigrid(cx, 3, 1, 3, 1, core.FP32)
+    op = core.LaplaceOperator(cx, 3, k, level, torch.float64)
+    tr = core.MGTransferCUDA(cx, 3, k, 1, level, torch.float64)
+    sm = core.PatchSmoother(op)
+    b = _dev(O.rhs_random(3, k, level))
+    f = _dev(rng(5).uniform(-1, 1, dg.n_dofs))
+    before = mg.solve_cg(b)[0].clone(), dg.solve_cg(f)[0].clone()
+    cx.close()
+    x, u = mg.solve_cg(b)[0], dg.solve_cg(f)[0]
+    y, c = torch.empty_like(b), torch.zeros((k * 4 + 1) ** 3, dtype=torch.float64,
+                                            device="cuda:0")
+    sm.vmult(y, b)
+    tr.restrict_and_add(level, c, y)
+    torch.cuda.synchronize()
+    assert torch.equal(x, before[0]) and torch.equal(u, before[1])
+    assert torch.isfinite(c).all()
+    del mg, dg, sm, tr
+    op.vmult(y, b)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y).all()
+    del op
+    cycle = [core.Context(0)]
+    cycle += [core.MultigridSolvers(cycle[0], 3, 1, 2, torch.float32),
+              core.DGMultigrid(cycle[0], 3, 1, 3, 0, core.FP32), cycle]
+    cycle[1].solve_cg(torch.ones(cycle[1].n_dofs, dtype=torch.float64, device="cuda:0"),
+                      raise_on_failure=False)
+    del cycle
+    gc.collect()
