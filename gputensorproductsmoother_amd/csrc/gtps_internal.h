@@ -304,12 +304,13 @@ namespace gtps
     // 1 = 8x8 / 256, 2 = 16x8 / 256; 3: by precision.  k = 7: 0 = 8x2 /
     // 512, 1 = 4x4 / 1024, 2 and 3 = 4x4 / 512
     int       vmult_tile = 3;
-    // 3D multiplicative sweeps: 1 = row kernel, two colours per launch; 0 =
-    // the per-colour kernels.  Measured on MI355X (us per sweep, row /
-    // per-colour): Q1 128^3 FP32 43 / 272, Q2 128^3 209 / 413, Q3 64^3 98 /
-    // 168 and FP64 156 / 252, Q4 32^3 55 / 377, Q5 32^3 FP64 191 / 599, Q7
-    // 32^3 262 / 542 and FP64 568 / 2746; smallest gains on coarse levels
-    // (Q3 8^3 23 / 32, Q7 8^3 64 / 68).
+    // 3D multiplicative sweeps: 1 = row kernel, two colours per launch,
+    // where it is faster (rows_pay in capi.hip); 0 = the per-colour kernels.
+    // Measured on MI355X in a graph (us per sweep, row / per colour): Q1 128^3
+    // FP32 38 / 272, Q2 128^3 206 / 412, Q3 64^3 93 / 160 and FP64 149 / 250,
+    // Q4 32^3 52 / 375, Q5 32^3 FP64 191 / 601, Q7 32^3 262 / 541 and FP64
+    // 568 / 2753; smallest gains on coarse levels (Q3 8^3 20 / 29, Q7 8^3 59 /
+    // 65).  DG sweeps and 2D additive sweeps: dg_rows_fit, additive2d_pays.
     int       row_sweeps = 1;
     // bumped by every successful gtps_set_tuning: HIP graphs captured under
     // an older generation are re-captured before their next replay

@@ -613,8 +613,9 @@ namespace gtps
       // interior lines per stage where registers and LDS leave at least two
       // work-groups a CU.  Measured on MI355X, us per sweep: k = 3 FP32 at
       // 64^3 98 with (16, 256) and 106 with (16, 512), at 32^3 36 and 27
-      // (a quarter of the rows: latency); k = 4 32^3 55 with (8, 512), 94
-      // with (4, 256); k = 7 FP32 32^3 262 with (4, 1024), 298 with
+      // (a quarter of the rows: latency; in a graph 93 and 25 as they are
+      // now); k = 4 32^3 55 with (8, 512), 94 with (4, 256); k = 7 FP32 32^3
+      // 262 with (4, 1024), 298 with
       // (4, 512), FP64 568 with (3, 512), 683 with (2, 512), 908 with
       // (3, 1024) (spills).
       constexpr bool d = sizeof(T) == 8;
