@@ -480,18 +480,18 @@ namespace gtps
   // Where three colours per launch are the faster form for nvec vectors at
   // once.  A row is one work-group whose time grows with n, while a colour
   // takes the time of one patch as long as its work-groups fit the 256 CUs at
-  // once; with the cheaper local solve of low degrees the launches saved
-  // decide on every mesh.  Measured on MI355X in a graph, us per sweep, rows /
+  // once; with the cheaper local solve of low degrees the launches saved decide
+  // on every mesh.  Measured on MI355X in a graph, us per sweep, rows /
   // colours, one vector (four): FP32 k = 1 5^3 58 / 96, 24^3 64 / 109 (67 /
-  // 162), k = 2 24^3 91 / 136 (97 / 211), k = 3
-  // 12^3 111 / 136, 20^3 135 / 152, k = 4 6^3 140 / 170 (141 / 173), 10^3 169
-  // / 171, 12^3 180 / 171 (184 / 182), 14^3 189 / 178 (197 / 235), 16^3 209 /
-  // 179 (215 / 256), 19^3 230 / 184 (241 / 431), 24^3 267 / 251 (289 / 717),
-  // 28^3 297 / 350, k = 5 11^3 247 / 253, 14^3 293 / 254 (306 / 428), 19^3
-  // 348 / 265 (368 / 956), 24^3 420 / 503, k = 6 9^3 323 / 358, 12^3 415 /
-  // 367; FP64 k = 1 24^3 74 / 121, k = 2 12^3 107 / 132, k = 3 12^3 154 / 160, 16^3 179 / 162 (184
-  // / 233), 19^3 188 / 165 (197 / 376), 24^3 210 / 229 (231 / 628), k = 4 8^3
-  // 211 / 209, 12^3 249 / 213, k = 5 7^3 361 / 365, 8^3 393 / 366.
+  // 162), k = 2 24^3 91 / 136 (97 / 211), k = 3 12^3 111 / 136, 20^3 135 / 152,
+  // k = 4 6^3 140 / 170 (141 / 173), 10^3 169 / 171, 12^3 180 / 171 (184 /
+  // 182), 14^3 189 / 178 (197 / 235), 16^3 209 / 179 (215 / 256), 19^3 230 /
+  // 184 (241 / 431), 24^3 267 / 251 (289 / 717), 28^3 297 / 350, k = 5 11^3 247
+  // / 253, 14^3 293 / 254 (306 / 428), 19^3 348 / 265 (368 / 956), 24^3 420 /
+  // 503, k = 6 9^3 323 / 358, 12^3 415 / 367; FP64 k = 1 24^3 74 / 121, k = 2
+  // 12^3 107 / 132, k = 3 12^3 154 / 160, 16^3 179 / 162 (184 / 233), 19^3 188
+  // / 165 (197 / 376), 24^3 210 / 229 (231 / 628), k = 4 8^3 211 / 209, 12^3
+  // 249 / 213, k = 5 7^3 361 / 365, 8^3 393 / 366.
   bool
   dg_rows_fit(int k, int prec, int n, int nvec)
   {
